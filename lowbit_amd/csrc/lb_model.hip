@@ -94,69 +94,208 @@ __global__ void qkv_rope_kernel(float *__restrict__ qkv, const float *__restrict
   }
 }
 
-// Causal grouped-query attention: query t (absolute position pos + t) of head h
-// against keys 0 .. pos + t of KV head h / (H / KV), softmax(q k^T / sqrt(D)) v
-// (src/lowbit/model.py:353-378). One workgroup of one wave per (token, head):
-// scores one key per lane into LDS, wave max and sum, then lane l owns output
-// elements l, l + 64, ... below D. q rows have stride qstride floats; out is [T, H D].
-template <int D>
-__global__ __launch_bounds__(kWave) void attention_kernel(const float *__restrict__ q, int qstride,
-                                                          const float *__restrict__ kc,
-                                                          const float *__restrict__ vc, int H, int KV,
-                                                          const int32_t *__restrict__ pos, int cap,
-                                                          float *__restrict__ out) {
-  extern __shared__ float sc[];  // [cap] scores, then [D] query
-  constexpr int DPL = (D + kWave - 1) / kWave;
-  const int t = blockIdx.x, h = blockIdx.y, lane = threadIdx.x;
-  const int kvh = h / (H / KV);
-  int S = *pos + t + 1;
-  S = S < cap ? S : cap;
-  float *qs = sc + cap;
-  const float *qr = q + (size_t)t * qstride + (size_t)h * D;
-  for (int e = lane; e < D; e += kWave) qs[e] = qr[e];
-  __syncthreads();
-  const float scale = 1.0f / sqrtf((float)D);
-  const float *kb = kc + (size_t)kvh * cap * D;
-  float mx = -INFINITY;
-  for (int s = lane; s < S; s += kWave) {
-    const float4 *kr = reinterpret_cast<const float4 *>(kb + (size_t)s * D);
-    float d = 0.0f;
-#pragma unroll 4
-    for (int e = 0; e < D / 4; e++) {
-      const float4 kv = kr[e];
-      d = __builtin_fmaf(qs[4 * e], kv.x, d);
-      d = __builtin_fmaf(qs[4 * e + 1], kv.y, d);
-      d = __builtin_fmaf(qs[4 * e + 2], kv.z, d);
-      d = __builtin_fmaf(qs[4 * e + 3], kv.w, d);
+// Causal grouped-query attention of a prompt: query t (absolute position pos + t) of
+// head h against keys 0 .. pos + t of KV head h / (H / KV), softmax(q k^T / sqrt(D)) v
+// (src/lowbit/model.py:353-378), in float32 on the float32 matrix cores
+// (v_mfma_f32_16x16x4_f32, 13.4 ns per SIMD: they bound it, 4 D products a key and
+// query). One workgroup of NW waves takes 16 queries of one head; its waves split the
+// keys in chunks of 16 KT (wave w: chunks w, w + NW, ...), so that the last queries'
+// long rows spread over a whole CU instead of being one wave's chain (heavy tiles start
+// first), and are merged once in LDS.
+//
+// Everything is computed transposed, scores^T = K Q^T and out^T = V^T P^T, so that a
+// lane keeps one query (lane % 16) throughout: the scores it gets from the first
+// product (keys 4 (lane / 16) + r, r = 0..3 of a 16-key tile) are, unmoved, the
+// operand of the second when slot lane / 16 of its step r stands for that key, and the
+// softmax's maximum, sum and rescale are per-lane values. K and V go from global
+// memory (16-byte loads in the operands' order) to registers with no LDS. In the d dimension the slots are free too: K and q elements
+// 16 j + 4 (lane / 16) + e feed step 4 j + e, and row i of output tile (b, x) is
+// d = 16 VW b + VW i + x, so that a lane's V loads and its outputs are contiguous.
+//
+// A chunk with keys some query may not see replaces their scores by -inf. Their V rows
+// must not reach the sum either, as 0 * inf or 0 * NaN: rows past every query's keys
+// are replaced by 0, and if a row that only some of the queries see is not finite, the
+// chunk's second product runs once per query with the rows that this query sees.
+//
+// Measured at D = 64 (one wave per query streaming all keys before -> now): 14 heads on
+// 2, 1000 tokens 270 -> 29.4 us (62 of 157 TFLOP/s; the rest is the softmax and waits
+// for L2), 384 tokens 50.8 -> 10.4, 16 tokens 4.1 both; 64 tokens behind 500 27 -> 10.5;
+// D = 128, 300 tokens, 8 heads on 4: 35.9 -> 12.2. 32-key chunks took 35.7 us at 1000
+// tokens (fewer waves fit), two query tiles a wave 32.0 there but 13.6 at 384 and 5.5 at
+// 16 tokens (half the workgroups), V loads one chunk ahead 34.8, four waves 31.0; at
+// D = 128 four waves (34 KiB of LDS) run 8 % faster than eight.
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));  // any float address
+typedef float f2u __attribute__((ext_vector_type(2), aligned(4)));
+
+template <int D, int NW>
+__global__ __launch_bounds__(NW *kWave) void attention_kernel(const float *__restrict__ q, int qstride,
+                                                              const float *__restrict__ kc,
+                                                              const float *__restrict__ vc, int T, int H, int KV,
+                                                              const int32_t *__restrict__ pos, int cap,
+                                                              float *__restrict__ out) {
+  constexpr int KT = D > 32 ? 1 : 2, CK = 16 * KT;          // 16-key tiles and keys per chunk
+  constexpr int DJ = D / 16;                                // 16-byte K loads per lane and tile
+  constexpr int VW = D >= 64 ? 4 : D / 16, VB = D / (16 * VW);  // floats per V load, loads per key
+  constexpr int PS = D + 4;                                 // LDS row of a wave's partial
+  using VV = std::conditional_t<VW == 4, f4u, f2u>;
+  __shared__ float part[NW][16][PS];
+  __shared__ float pm[NW][16], pl[NW][16];
+  const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int c = lane & 15, g = lane >> 4;
+  const int h = blockIdx.x, kvh = h / (H / KV);
+  const int t0 = (int)(gridDim.y - 1 - blockIdx.y) * 16;
+  const float *kb = kc + (size_t)kvh * cap * D, *vb = vc + (size_t)kvh * cap * D;
+  const int p0 = *pos;
+  // keys of the first and last query of the tile, and of this lane's
+  const auto keys_of = [&](int t) { return min(p0 + min(t, T - 1) + 1, cap); };
+  const int Smin = keys_of(t0), Smax = keys_of(t0 + 15), S = keys_of(t0 + c);
+  f4u qf[DJ];
+  const float *qr = q + (size_t)min(t0 + c, T - 1) * qstride + (size_t)h * D + 4 * g;
+#pragma unroll
+  for (int j = 0; j < DJ; j++) qf[j] = *reinterpret_cast<const f4u *>(qr + 16 * j);
+  // exp((s - max) / sqrt(D)) as exp2(s cs - max cs), max cs rounded once for all
+  const float cs = 1.4426950408889634f / sqrtf((float)D);
+  float m = -INFINITY, l = 0.0f;  // running maximum times cs, sum
+  v4f acc[VB][VW];
+#pragma unroll
+  for (int b = 0; b < VB; b++)
+#pragma unroll
+    for (int y = 0; y < VW; y++) acc[b][y] = v4f{0.f, 0.f, 0.f, 0.f};
+  f4u kf[KT][DJ];
+  VV vf[KT][4][VB];
+  // rows clamped below cap: every address is inside the cache
+  const auto load_k = [&](int k0) {
+#pragma unroll
+    for (int a = 0; a < KT; a++) {
+      const float *kr = kb + (size_t)min(k0 + 16 * a + c, cap - 1) * D + 4 * g;
+#pragma unroll
+      for (int j = 0; j < DJ; j++) kf[a][j] = *reinterpret_cast<const f4u *>(kr + 16 * j);
     }
-    d *= scale;
-    sc[s] = d;
-    mx = fmaxf(mx, d);
+  };
+  if (CK * wave < Smax) load_k(CK * wave);
+  for (int k0 = CK * wave; k0 < Smax; k0 += CK * NW) {
+#pragma unroll
+    for (int a = 0; a < KT; a++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const float *vr = vb + (size_t)min(k0 + 16 * a + 4 * g + r, cap - 1) * D + VW * c;
+#pragma unroll
+        for (int b = 0; b < VB; b++) vf[a][r][b] = *reinterpret_cast<const VV *>(vr + 16 * VW * b);
+      }
+    v4f s[KT];
+#pragma unroll
+    for (int a = 0; a < KT; a++) s[a] = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < DJ; j++)
+#pragma unroll
+      for (int e = 0; e < 4; e++)
+#pragma unroll
+        for (int a = 0; a < KT; a++) s[a] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[a][j][e], qf[j][e], s[a], 0, 0, 0);
+    if (k0 + CK * NW < Smax) load_k(k0 + CK * NW);
+    const bool edge = k0 + CK > Smin;  // wave-uniform: some query does not see the whole chunk
+    bool apart = false;
+    if (edge) {
+      float bad = 0.0f;
+#pragma unroll
+      for (int a = 0; a < KT; a++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          const int k = k0 + 16 * a + 4 * g + r;
+          s[a][r] = k < S ? s[a][r] : -INFINITY;
+#pragma unroll
+          for (int b = 0; b < VB; b++)
+#pragma unroll
+            for (int y = 0; y < VW; y++) {
+              vf[a][r][b][y] = k < Smax ? vf[a][r][b][y] : 0.0f;
+              bad = __builtin_fmaf(vf[a][r][b][y], 0.0f, bad);  // NaN if not finite
+            }
+        }
+      apart = __any(bad != bad);
+    }
+    float mx = -INFINITY;
+#pragma unroll
+    for (int a = 0; a < KT; a++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) mx = fmaxf(mx, s[a][r]);
+    mx = fmaxf(mx, __shfl_xor(mx, 16));
+    mx = fmaxf(mx, __shfl_xor(mx, 32));
+    const float mnew = fmaxf(m, mx * cs);
+    const float ref = mnew == -INFINITY ? 0.0f : mnew;  // no key yet: weights exp2(-inf) = 0
+    const float alpha = __builtin_amdgcn_exp2f(m - ref);
+    m = mnew;
+    float sum = 0.0f;
+#pragma unroll
+    for (int a = 0; a < KT; a++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        s[a][r] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[a][r], cs, -ref));
+        sum += s[a][r];
+      }
+    l = __builtin_fmaf(l, alpha, sum);  // this lane's keys; the lanes are added at the end
+#pragma unroll
+    for (int b = 0; b < VB; b++)
+#pragma unroll
+      for (int y = 0; y < VW; y++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) acc[b][y][r] *= alpha;
+    if (!apart) {
+#pragma unroll
+      for (int a = 0; a < KT; a++)
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+#pragma unroll
+          for (int b = 0; b < VB; b++)
+#pragma unroll
+            for (int y = 0; y < VW; y++)
+              acc[b][y] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[a][r][b][y], s[a][r], acc[b][y], 0, 0, 0);
+    } else {
+      for (int i = 0; i < 16; i++) {  // query i of the tile alone, with the rows it sees
+        const int Si = keys_of(t0 + i);
+#pragma unroll
+        for (int b = 0; b < VB; b++)
+#pragma unroll
+          for (int y = 0; y < VW; y++) {
+            v4f o = acc[b][y];
+#pragma unroll
+            for (int a = 0; a < KT; a++)
+#pragma unroll
+              for (int r = 0; r < 4; r++)
+                o = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                    k0 + 16 * a + 4 * g + r < Si ? (float)vf[a][r][b][y] : 0.0f, s[a][r], o, 0, 0, 0);
+#pragma unroll
+            for (int r = 0; r < 4; r++) acc[b][y][r] = c == i ? o[r] : acc[b][y][r];
+          }
+      }
+    }
   }
-  mx = wave_max(mx);
-  float sum = 0.0f;
-  for (int s = lane; s < S; s += kWave) {
-    const float e = expf(sc[s] - mx);
-    sc[s] = e;
-    sum += e;
+  // ---- the waves' partial sums, merged in wave order
+  l += __shfl_xor(l, 16);
+  l += __shfl_xor(l, 32);
+  if (g == 0) {
+    pm[wave][c] = m;
+    pl[wave][c] = l;
   }
-  sum = wave_sum(sum);
+#pragma unroll
+  for (int b = 0; b < VB; b++)
+#pragma unroll
+    for (int r = 0; r < 4; r++)
+#pragma unroll
+      for (int y = 0; y < VW; y++) part[wave][c][16 * VW * b + VW * (4 * g + r) + y] = acc[b][y][r];
   __syncthreads();
-  const float inv = 1.0f / sum;
-  const float *vb = vc + (size_t)kvh * cap * D;
-  const bool own = D >= kWave || lane < D;  // D = 32: lanes 32..63 hold no output
-  const int l = own ? lane : 0;
-  float acc[DPL];
+  for (int e = threadIdx.x; e < 16 * D; e += NW * kWave) {
+    const int i = e / D, d = e % D, t = t0 + i;
+    if (t >= T) break;
+    float M = pm[0][i];
 #pragma unroll
-  for (int j = 0; j < DPL; j++) acc[j] = 0.0f;
-  for (int s = 0; s < S; s++) {
-    const float ps = sc[s];
+    for (int w = 1; w < NW; w++) M = fmaxf(M, pm[w][i]);
+    float num = 0.0f, den = 0.0f;
 #pragma unroll
-    for (int j = 0; j < DPL; j++) acc[j] = __builtin_fmaf(ps, vb[(size_t)s * D + l + kWave * j], acc[j]);
-  }
-  if (own) {
-#pragma unroll
-    for (int j = 0; j < DPL; j++) out[(size_t)t * H * D + (size_t)h * D + l + kWave * j] = acc[j] * inv;
+    for (int w = 0; w < NW; w++) {
+      const float f = __builtin_amdgcn_exp2f(pm[w][i] - M);  // 0 for a wave that saw no key
+      num = __builtin_fmaf(part[w][i][d], f, num);
+      den = __builtin_fmaf(pl[w][i], f, den);
+    }
+    out[(size_t)t * H * D + (size_t)h * D + d] = num / den;
   }
 }
 
@@ -506,17 +645,15 @@ hipError_t launch_qkv_rope(float *qkv, const float *bias, int T, int H, int KV, 
 
 hipError_t launch_attention(const float *q, int qstride, const float *kc, const float *vc, int T, int H, int KV, int D,
                             const int32_t *pos, int cap, float *out, hipStream_t s) {
-  const size_t lds = ((size_t)cap + D) * sizeof(float);
-  if (D == 32)
-    hipLaunchKernelGGL(attention_kernel<32>, dim3(T, H), dim3(kWave), lds, s, q, qstride, kc, vc, H, KV, pos, cap, out);
-  else if (D == 64)
-    hipLaunchKernelGGL(attention_kernel<64>, dim3(T, H), dim3(kWave), lds, s, q, qstride, kc, vc, H, KV, pos, cap, out);
-  else if (D == 128)
-    hipLaunchKernelGGL(attention_kernel<128>, dim3(T, H), dim3(kWave), lds, s, q, qstride, kc, vc, H, KV, pos, cap,
+  auto go = [&](auto kern, int nw) {
+    hipLaunchKernelGGL(kern, dim3(H, (T + 15) / 16), dim3(nw * kWave), 0, s, q, qstride, kc, vc, T, H, KV, pos, cap,
                        out);
-  else
-    return hipErrorInvalidValue;
-  return hipGetLastError();
+    return hipGetLastError();
+  };
+  if (D == 32) return go(attention_kernel<32, 8>, 8);
+  if (D == 64) return go(attention_kernel<64, 8>, 8);
+  if (D == 128) return go(attention_kernel<128, 4>, 4);
+  return hipErrorInvalidValue;
 }
 
 hipError_t launch_swiglu(const float *gu, int T, int I, float *out, hipStream_t s) {
