@@ -231,8 +231,9 @@ size_t lbd_bf16x3_workspace_bytes(int M, int Kp);
  * activations, then the slices' partial outputs, added by one more launch in slice
  * order. A workspace of this size (or NULL) takes the split, one of
  * lbd_bf16x3_workspace_bytes the unsplit GEMM; both meet the same bound, not the
- * same bits. Equals lbd_bf16x3_workspace_bytes rounded up to 256 where no split is
- * taken; 0 for an invalid argument. (No reference counterpart: the reference's
+ * same bits. (Shapes of many rows that run as prompt GEMMs take no split and leave the
+ * room for it unused.) Equals lbd_bf16x3_workspace_bytes rounded up to 256 where no
+ * split is taken; 0 for an invalid argument. (No reference counterpart: the reference's
  * GEMMs take no workspace.) */
 size_t lbd_bf16x3_workspace_bytes_split(int kind, int M, int N, int Kp);
 /* ---- "t16f8": int4 g128 weights for lbd_gemm_w4a16 on the matrix cores with the
@@ -269,7 +270,10 @@ int lbd_mxfp4_t16_bytes(int N, int Kp, size_t *qwt_bytes, size_t *et_bytes);
 int lbd_repack_mxfp4_t16(const uint8_t *qw, const uint8_t *e8m0, int N, int Kp,
                          uint8_t *qwt, uint8_t *et, void *stream);
 /* y = x . w^T as lbd_gemm_mxfp4 on t16 weights, the bf16 matrix-core path of
- * lbd_gemm_w4a16_t16 (block scales 2^(e - 127) exact; E8M0 255 gives NaN) */
+ * lbd_gemm_w4a16_t16 (block scales 2^(e - 127) exact; E8M0 255 gives NaN). With many
+ * rows it runs on the MX matrix instruction instead, which takes the weights as they
+ * are: the activations become 7 six-bit digits per element (more beside an outlier that
+ * they do not reach), within the same workspace. */
 int lbd_gemm_mxfp4_t16(const float *x, int M, int Kp, const uint8_t *qwt,
                        const uint8_t *et, int N, float *y, const lb_params *p,
                        void *workspace, size_t workspace_bytes, void *stream);

@@ -257,16 +257,21 @@ int run_bf3(int fmt, const lbk::GemmArgs &a0, char *ws, hipStream_t s, bool f8 =
   lbk::GemmArgs a = a0;
   a.x3 = reinterpret_cast<const uint4 *>(ws);
   hipError_t e;
+  lbk::PromptTile tile;
+  const bool prompt = lbk::prompt_tile_for(fmt, a.M, a.N, a.Kp, cus, &tile);
   if (fmt == lbk::F_W4A16) {
     // two float16 terms per row and its exponent (within the bf16x3 workspace)
     int *xexp = reinterpret_cast<int *>(ws + lbk::x2h_exp_offset(a.M, a.Kp));
     a.xexp = xexp;
     e = lbk::launch_split2h(a.x, a.M, a.Kp, reinterpret_cast<uint4 *>(ws), xexp, s);
+  } else if (prompt) {
+    e = lbk::launch_split_digits(a.x, a.M, a.Kp, ws, s);
   } else {
     e = lbk::launch_split3(fmt, a.x, a.M, a.Kp, reinterpret_cast<uint4 *>(ws), s);
   }
   if (e != hipSuccess) return fail_hip(e, "activation split launch");
-  e = lbk::launch_bf3_gemm(fmt, a, cus, s, f8);
+  if (!prompt) e = lbk::launch_bf3_gemm(fmt, a, cus, s, f8);
+  else e = lbk::launch_mxfp4_prompt(a, tile, s);
   if (e != hipSuccess) return fail_hip(e, "bf16x3 GEMM launch");
   return ok(LB_ISA_GFX950_MFMA);
 }

@@ -142,6 +142,18 @@ inline size_t tiled_asum_bytes(int M, int Kp) { return (size_t)((M + 15) / 16) *
 // int8 MFMA W4A8 on quantized activations; with `out` non-null it writes the
 // exact int32 group accumulators [M, N, G] instead of Y.
 hipError_t launch_w4a8_mfma(const GemmArgs &a, int32_t *out, int num_cus, hipStream_t s);
+// Prompt GEMMs (lb_prompt.hip): workgroup tile of 16 tm rows x 64 wn columns.
+struct PromptTile {
+  int tm = 0, wn = 0;
+};
+// Whether a t16 GEMM of this shape runs faster on them than on the batch kernels, and how.
+bool prompt_tile_for(int fmt, int M, int N, int Kp, int num_cus, PromptTile *out);
+// MXFP4 with many rows (lb_prompt.hip): the activations as kDigits E2M3 digits per
+// element (digit_bytes(M, Kp) bytes, within x3_bytes), the GEMM on them and t16 weights.
+constexpr int kDigits = 7;
+size_t digit_bytes(int M, int Kp);
+hipError_t launch_split_digits(const float *x, int M, int Kp, void *out, hipStream_t s);
+hipError_t launch_mxfp4_prompt(const GemmArgs &a, PromptTile t, hipStream_t s);
 // fp32 MFMA W4A16 / MXFP4.
 hipError_t launch_f32_mfma(int fmt, const GemmArgs &a, hipStream_t s);
 // exact int32 group accumulators through the VALU dot4 arithmetic of the GEMV.

@@ -1,0 +1,355 @@
+// Prompt GEMMs (many activation rows) on the matrix cores: Y[M,N] = X[M,Kp] . W[N,Kp]^T
+// with the weights in the t16 tile layout and the activations in the operand tiles that
+// the quantizer and the split kernels write (lb_kernels.hip).
+//
+// The batch kernels of lb_kernels.hip hold a few row blocks in registers and stream the
+// weights past them, every weight tile ending in a reduction over the workgroup's waves;
+// with hundreds of rows that reads and decodes the weights once per 16-64 rows and
+// reduces far too often. Here a workgroup owns a tile of 16 TM rows x 16 WN NW columns
+// of Y and walks K group by group:
+//   * activations: the stage of the next group goes straight to LDS (buffer loads with
+//     the LDS flag, no registers) while the current one is consumed from the other
+//     buffer; the tiles are in operand order, so every LDS access is a conflict-free
+//     16-byte read of 64 consecutive lanes. One barrier a group.
+//   * weights: each wave owns WN 16-row subtiles and loads their tiles, scales and
+//     zero-points for the next group into registers; they are decoded once per TM row
+//     blocks and never pass through LDS.
+//   * sums stay in the wave's registers for all of K: no reduction, no second pass.
+#include <algorithm>
+#include <cmath>
+
+#include "lb_device.h"
+#include "lb_internal.h"
+
+namespace lbk {
+
+constexpr int kPWaves = 4, kPThreads = kPWaves * kWave;
+
+// A stage's two buffers are separate objects (not one array indexed by parity), so that
+// the compiler sees that reads of one do not depend on the loads still filling the other.
+__device__ __forceinline__ void lds_load16(Rsrc r, char *dst, uint32_t voff, uint32_t soff) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void *)dst, 16, (int)voff, (int)soff,
+                                           0, 0);
+}
+__device__ __forceinline__ void lds_load4(Rsrc r, char *dst, uint32_t voff, uint32_t soff) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void *)dst, 4, (int)voff, (int)soff, 0,
+                                           0);
+}
+
+// This wave's loads but the last LATER have arrived, those to LDS too (which a barrier
+// alone does not wait for), and every wave is done with the stage before. Loads retire in
+// order, and every wave issues the same number a group, so LATER = the loads of the groups
+// after the one about to run.
+template <int LATER>
+__device__ __forceinline__ void stage_ready() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LATER) : "memory");
+  __syncthreads();
+}
+
+// Tile of this workgroup: workgroups go to the 8 XCDs in turn, each XCD takes a
+// contiguous run of tiles, in bands of four row tiles walked column by column, so that
+// the tiles it works on at one time (32 or more) form a block whose weights are shared
+// by four of them and whose activations by eight, in its L2. False past the last tile.
+__device__ __forceinline__ bool prompt_tile(int mt, int nt, int &tm, int &tn) {
+  const int total = mt * nt, per = (total + 7) / 8;
+  const int t = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
+  const int band = t / (4 * nt), in = t - band * 4 * nt, rows = min(4, mt - 4 * band);
+  tn = in / rows;
+  tm = 4 * band + in - tn * rows;
+  return (int)(blockIdx.x / 8) < per && t < total;
+}
+template <typename Kern>
+static hipError_t launch_prompt(Kern kern, const GemmArgs &a, PromptTile t, hipStream_t s) {
+  const int mt = (a.M + 16 * t.tm - 1) / (16 * t.tm), nt = (a.N + 64 * t.wn - 1) / (64 * t.wn);
+  const unsigned grid = 8u * (unsigned)(((size_t)mt * nt + 7) / 8);
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(kPThreads), 0, s, a, mt, nt);
+  return hipGetLastError();
+}
+
+// ============================================================ MXFP4
+//
+// The MX matrix instruction (v_mfma_scale_f32_16x16x128_f8f6f4) takes E2M1 weights and
+// their E8M0 block scales as they are, a 128-element group per instruction, at four
+// times the bf16 rate when the other operand is 6 bits wide. So the weights need no
+// decode at all, and each activation becomes kDigits signed digits of E2M3, which holds
+// every integer of [-16, 16] (times 1/8): with 2^ex above the largest |x| of its block
+// of 32, x 2^(4 - ex) = d1 + d2 2^-5 + d3 2^-10 ..., d1 = rint of it, and so on with the
+// exact remainders, the powers of two in the activations' own E8M0 scales. Seven digits
+// hold every element within 2^10 of its block's largest exactly and the others to
+// 2^-35 of 2^ex; a block where four or more elements lose bits to that (an outlier among
+// ordinary elements; normal ones hardly ever do, 2e-7 of blocks) is marked, and the GEMM makes
+// the further digits it takes from the activations themselves. Products and their sums over a group are exact up to the float32
+// accumulator. The leading digits add to one accumulator and the other six, 2^-5 of its
+// size, to a second, so that Y sees one float32 rounding per group.
+//
+// Digit tile of (row block, group, digit): lane 16 q + c holds row c, block 4 g + q, slots
+// 2 j / 2 j + 1 = elements j / j + 16 (the nibbles of byte j of the packed weights),
+// 24 bytes as 16 (1 KiB for the wave) then 8 (512 B); then 8 bytes per lane, the digits'
+// E8M0 scales and the mark.
+constexpr int kDigitTile = kWave * 24, kDigitBlock = kDigits * kDigitTile + kWave * 8;
+static_assert(kDigitBlock == 11 * 1024, "the GEMM stages whole KiB");
+size_t digit_bytes(int M, int Kp) { return (size_t)((M + 15) / 16) * ((Kp + 127) / 128) * kDigitBlock; }
+
+typedef float v16f __attribute__((ext_vector_type(16)));
+typedef unsigned int v6u __attribute__((ext_vector_type(6)));
+typedef int v8i __attribute__((ext_vector_type(8)));
+typedef unsigned int v2u __attribute__((ext_vector_type(2)));
+
+// A lane's block of 32 activations as digits: lo and hi hold its halves, times 2^(4 - ex),
+// less the digits taken so far, in units of the next one.
+struct DigitBlock {
+  v16f lo, hi;
+  int e8;    // biased exponent of the next digit's scale
+  bool bad;  // holds an infinity or NaN
+
+  __device__ __forceinline__ void load(const float *x, int M, int Kp, int row, int b) {
+    const Rsrc rx = make_rsrc(x, (uint32_t)((size_t)M * Kp * 4));
+    const uint32_t off = row < M && 32 * b < Kp ? (uint32_t)(((size_t)row * Kp + 32 * b) * 4) : 0xFFFFFF00u;
+    uint32_t top = 0;
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      const float4 t = ld_f4(rx, off + 16 * i);
+      const float e[4] = {t.x, t.y, t.z, t.w};
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        top = max(top, __float_as_uint(e[k]) & 0x7FFFFFFFu);
+        if (i < 4) lo[4 * i + k] = e[k];
+        else hi[4 * (i - 4) + k] = e[k];
+      }
+    }
+    int ex = 0;
+    (void)frexpf(__uint_as_float(top), &ex);  // top < 2^ex
+    bad = top >= 0x7F800000u;
+#pragma unroll
+    for (int i = 0; i < 16; i++) lo[i] = ldexpf(lo[i], 4 - ex), hi[i] = ldexpf(hi[i], 4 - ex);
+    e8 = 127 + ex - 4 + 3;  // the first digit counts units of 2^(ex - 4), the tiles hold eighths
+  }
+  // the next digits, six bits each; zeros below the smallest scale
+  __device__ __forceinline__ v6u next() {
+    v16f dl, dh;
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+      dl[i] = __builtin_rintf(lo[i]);
+      dh[i] = __builtin_rintf(hi[i]);
+      lo[i] = (lo[i] - dl[i]) * 32.0f;
+      hi[i] = (hi[i] - dh[i]) * 32.0f;
+      if (e8 < 0) dl[i] = 0.0f, dh[i] = 0.0f;
+    }
+    e8 -= 5;
+    return __builtin_amdgcn_cvt_scalef32_2xpk16_fp6_f32(dl, dh, 8.0f);
+  }
+  // elements that the digits so far do not hold exactly
+  __device__ __forceinline__ int inexact() const {
+    int n = 0;
+#pragma unroll
+    for (int i = 0; i < 16; i++) n += (lo[i] != 0.0f) + (hi[i] != 0.0f);
+    return n;
+  }
+};
+
+// One wave per (row block, group), one lane per (row, block). An infinity or NaN makes
+// its block's scales NaN (255), so the row's outputs are NaN, as in the bf16 split.
+__global__ __launch_bounds__(kPThreads) void split_digits_kernel(const float *__restrict__ x, int M, int Kp,
+                                                                 char *__restrict__ out) {
+  const int lane = threadIdx.x & (kWave - 1), G = (Kp + 127) / 128, mblocks = (M + 15) / 16;
+  const size_t item = (size_t)blockIdx.x * kPWaves + threadIdx.x / kWave;
+  if (item >= (size_t)mblocks * G) return;  // whole waves only
+  const int mb = (int)(item % mblocks), g = (int)(item / mblocks);
+  DigitBlock d;
+  d.load(x, M, Kp, 16 * mb + (lane & 15), 4 * g + (lane >> 4));
+  char *dst = out + item * kDigitBlock;
+  uint32_t sc[2] = {0, 0};
+#pragma unroll
+  for (int t = 0; t < kDigits; t++) {
+    sc[t / 4] |= (d.bad ? 255u : (uint32_t)max(d.e8, 0)) << (8 * (t % 4));
+    const v6u p = d.next();
+    *reinterpret_cast<uint4 *>(dst + t * kDigitTile + lane * 16) = make_uint4(p[0], p[1], p[2], p[3]);
+    *reinterpret_cast<uint2 *>(dst + t * kDigitTile + 1024 + lane * 8) = make_uint2(p[4], p[5]);
+  }
+  if (!d.bad && d.inexact() >= 4) sc[1] |= 1u << 24;
+  *reinterpret_cast<uint2 *>(dst + kDigits * kDigitTile + lane * 8) = make_uint2(sc[0], sc[1]);
+}
+
+hipError_t launch_split_digits(const float *x, int M, int Kp, void *out, hipStream_t s) {
+  const size_t items = (size_t)((M + 15) / 16) * ((Kp + 127) / 128);
+  hipLaunchKernelGGL(split_digits_kernel, dim3((unsigned)((items + kPWaves - 1) / kPWaves)), dim3(kPThreads), 0, s, x,
+                     M, Kp, static_cast<char *>(out));
+  return hipGetLastError();
+}
+
+// c + x . w: six-bit digits with scale byte `sel` of sx, E2M1 weights with scale sw.
+__device__ __forceinline__ v4f mx_product(int sel, v8i x, int sx, uint4 w4, int sw, v4f c) {
+  const v8i w = {(int)w4.x, (int)w4.y, (int)w4.z, (int)w4.w, 0, 0, 0, 0};
+  switch (sel) {  // a constant once the callers are unrolled
+    case 0: return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(x, w, c, 2, 4, 0, sx, 0, sw);
+    case 1: return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(x, w, c, 2, 4, 1, sx, 0, sw);
+    case 2: return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(x, w, c, 2, 4, 2, sx, 0, sw);
+    default: return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(x, w, c, 2, 4, 3, sx, 0, sw);
+  }
+}
+
+template <int TM, int WN>
+__global__ __launch_bounds__(kPThreads, 2) void mxfp4_prompt_kernel(GemmArgs a, int mt, int nt) {
+  constexpr int SK = TM * kDigitBlock / 1024;  // KiB of a stage
+  constexpr int PW = (SK + kPWaves - 1) / kPWaves;
+  __shared__ __align__(16) char xs0[SK * 1024], xs1[SK * 1024], xs2[SK * 1024];
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int q = lane >> 4, c = lane & 15;
+  const int M = a.M, N = a.N, Kp = a.Kp, G = (Kp + 127) / 128, G4 = t16_groups(Kp), S = (N + 15) / 16;
+  int tm, tn;
+  if (!prompt_tile(mt, nt, tm, tn)) return;
+  const int mb0 = tm * TM, s0 = (tn * kPWaves + wave) * WN;
+  const uint32_t mblocks = (uint32_t)((M + 15) / 16);
+  const Rsrc rx = make_rsrc(a.x3, (uint32_t)min((size_t)mblocks * G * kDigitBlock, (size_t)0xFFFFFFF0u));
+  const Rsrc rw = make_rsrc(a.qw, (uint32_t)min(t16_qw_bytes(N, Kp), (size_t)0xFFFFFFF0u));
+  const Rsrc re = make_rsrc(a.e8m0, (uint32_t)t16_e8m0_bytes(N, Kp));
+
+  struct Weights {
+    uint4 w[WN];
+    uint32_t e[WN];
+  } w0, w1, w2;
+  // load `op` of this wave for group g: the first PW copy its share of the stage (row blocks
+  // are consecutive within a group, so a stage is one run of KiB; past the last row block
+  // it reads the next group's, rows that are not stored, or zeros at the end), the others
+  // load its subtiles' weights and scales (past the last subtile: its columns are not stored)
+  constexpr int OPS = PW + 2 * WN;
+  const auto load = [&](int op, char *xd, Weights &n, int g) {
+    if (op < PW) {
+      const int t = min(wave * PW + op, SK - 1);
+      lds_load16(rx, xd + t * 1024, (uint32_t)lane * 16u + ((uint32_t)g * mblocks + (uint32_t)mb0) * (uint32_t)kDigitBlock +
+                     (uint32_t)t * 1024u, 0);
+    } else if (op < OPS) {
+      const int j = (op - PW) >> 1;
+      const uint32_t sj = (uint32_t)min(s0 + j, S - 1);
+      if ((op - PW) & 1) n.e[j] = __builtin_amdgcn_raw_buffer_load_b8(re, lane, (int)((sj * G4 + g) * 64u), 0);
+      else n.w[j] = ld_b128(rw, (uint32_t)lane * 16u, (sj * G4 + g) * 1024u);
+    }
+  };
+  v4f hi[TM][WN], lo[TM][WN];
+#pragma unroll
+  for (int i = 0; i < TM; i++)
+#pragma unroll
+    for (int j = 0; j < WN; j++) hi[i][j] = v4f{0.f, 0.f, 0.f, 0.f}, lo[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
+
+  // One group, with the loads of the one after the next between its products. A product
+  // occupies the matrix core for 16 cycles and the wave's issue for 8, so
+  // what is issued one by one between products costs nothing, and in clumps its whole time;
+  // every slot is pinned, as the scheduler would make clumps (and sink the loads to the end).
+  const auto group = [&](const char *xd, const Weights &n, char *nxd, Weights &nn, int g) {
+    constexpr int K = TM * kDigits;  // step k: row block k / kDigits, digit k % kDigits
+    v4i xa[3];
+    v2u xb[3], sc[2];
+    const auto read_a = [&](int k) {
+      xa[k % 3] = *reinterpret_cast<const v4i *>(xd + (k / kDigits) * kDigitBlock + (k % kDigits) * kDigitTile + lane * 16);
+    };
+    const auto read_b = [&](int k) {
+      const char *blk = xd + (k / kDigits) * kDigitBlock;
+      xb[k % 3] = *reinterpret_cast<const v2u *>(blk + (k % kDigits) * kDigitTile + 1024 + lane * 8);
+      if (k % kDigits == 0)
+        sc[(k / kDigits) & 1] = *reinterpret_cast<const v2u *>(blk + kDigits * kDigitTile + lane * 8);
+    };
+    read_a(0);
+    read_b(0);
+    read_a(1);
+    read_b(1);
+    int op = 0;
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+      const int i = k / kDigits, t = k % kDigits;
+      const v8i x = {xa[k % 3][0], xa[k % 3][1], xa[k % 3][2], xa[k % 3][3], (int)xb[k % 3][0], (int)xb[k % 3][1], 0, 0};
+#pragma unroll
+      for (int j = 0; j < WN; j++) {
+        v4f &o = t == 0 ? hi[i][j] : lo[i][j];
+        o = mx_product(t & 3, x, (int)sc[i & 1][t >> 2], n.w[j], (int)n.e[j], o);
+        __builtin_amdgcn_sched_barrier(0);
+        if (j == 0 && k + 2 < K) read_a(k + 2);
+        if (j == 1 && k + 2 < K) read_b(k + 2);
+        if (j >= 2) load(op++, nxd, nn, min(g + 2, G - 1));
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    static_assert(K * (WN - 2) >= OPS, "every load has a slot");
+#pragma unroll
+    for (int i = 0; i < TM; i++) {
+      if (!__any((int)(sc[i & 1][1] >> 24))) continue;
+      DigitBlock d;
+      d.load(a.x, M, Kp, 16 * (mb0 + i) + c, 4 * g + q);
+#pragma unroll 1
+      for (int t = 0; t < kDigits; t++) (void)d.next();
+      while (__any(!d.bad && d.e8 >= 0 && d.inexact() > 0)) {
+        const int sx = d.bad ? 255 : max(d.e8, 0);
+        const v6u p = d.next();
+        const v8i x = {(int)p[0], (int)p[1], (int)p[2], (int)p[3], (int)p[4], (int)p[5], 0, 0};
+#pragma unroll
+        for (int j = 0; j < WN; j++) lo[i][j] = mx_product(0, x, sx, n.w[j], (int)n.e[j], lo[i][j]);
+      }
+    }
+  };
+  // two groups are in flight ahead of the one that runs
+#pragma unroll
+  for (int op = 0; op < OPS; op++) load(op, xs0, w0, 0);
+#pragma unroll
+  for (int op = 0; op < OPS; op++) load(op, xs1, w1, min(1, G - 1));
+  const auto step = [&](const char *xd, const Weights &n, char *nxd, Weights &nn, int g) {
+    stage_ready<OPS>();
+    group(xd, n, nxd, nn, g);
+  };
+  for (int g = 0; g < G; g += 3) {
+    step(xs0, w0, xs2, w2, g);
+    if (g + 1 < G) step(xs1, w1, xs0, w0, g + 1);
+    if (g + 2 < G) step(xs2, w2, xs1, w1, g + 2);
+  }
+  stage_ready<0>();  // no load to LDS outlives the workgroup
+#pragma unroll
+  for (int i = 0; i < TM; i++) {
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int m = (mb0 + i) * 16 + 4 * q + r;
+      if (m >= M) continue;
+#pragma unroll
+      for (int j = 0; j < WN; j++) {
+        const int n = 16 * (s0 + j) + c;
+        if (n < N) a.y[(size_t)m * N + n] = hi[i][j][r] + lo[i][j][r];
+      }
+    }
+  }
+}
+
+hipError_t launch_mxfp4_prompt(const GemmArgs &a, PromptTile t, hipStream_t s) {
+  if (!a.wt16 || !a.x3) return hipErrorInvalidValue;
+  if (t.tm == 1) return launch_prompt(mxfp4_prompt_kernel<1, 4>, a, t, s);
+  return launch_prompt(mxfp4_prompt_kernel<2, 4>, a, t, s);
+}
+
+// ============================================================ dispatch
+//
+// Where these kernels beat the batch kernels, from both sides' times (us) at 56 shapes of
+// 80-1024 rows, N 300-11008, K 896-11008 with the weights warm. A tile walks K serially:
+// a launch that leaves each CU one workgroup or less takes (a little more than) G times
+// its time per group however few rows there are, while the batch kernels' time falls with
+// the work; so the line is drawn in 16 x 16 tiles of Y per CU, T.
+//   MXFP4  0.72 us a group; 0.55 with 16-row tiles, taken while they fill one round of the
+//          CUs (256 x 4096 x 4096 29.5 -> 26.0). Wins from T = 12 at every K
+//          (192 x 4096 x 4096 38.8 -> 25.9, x 11008 87.8 -> 56.2, 1024 x 4096 x 4096 179 ->
+//          61; 128 rows 19.5 against 25.0, not taken).
+// Few rows (32 and less) stay with the batch kernels, which are built for them.
+bool prompt_tile_for(int fmt, int M, int N, [[maybe_unused]] int Kp, int num_cus, PromptTile *out) {
+  if (M <= 32) return false;
+  const double cus = num_cus > 0 ? num_cus : 256;
+  const double T = (double)((M + 15) / 16) * ((N + 15) / 16) / cus;
+  const auto rounds = [&](int tm, int wn) {
+    return (double)((M + 16 * tm - 1) / (16 * tm)) * ((N + 64 * wn - 1) / (64 * wn)) / cus;
+  };
+  PromptTile t;
+  if (fmt == F_MXFP4) {
+    if (T < 12) return false;
+    t = PromptTile{rounds(1, 4) <= 1 ? 1 : 2, 4};
+  } else {
+    return false;
+  }
+  *out = t;
+  return true;
+}
+
+}  // namespace lbk

@@ -1,0 +1,53 @@
+"""The prompt GEMMs (lb_prompt.hip) at the edges of their tiles (GPU): row blocks and
+subtiles past the matrix, one and an odd number of K groups, the stage buffers with every
+number of groups left over, the largest zero-points, against the float64 oracle within the
+bounds that the batch kernels' tests use."""
+import numpy as np
+import pytest
+
+import lowbit_amd as lb
+from lowbit_amd import kernels as K
+from oracle import reference as O
+
+pytestmark = pytest.mark.gpu
+
+# M, N, K: ragged M and N, 1, 2, 3, 7 and 8 groups; 13 or more 16 x 16 tiles of Y per CU,
+# where every format takes these kernels
+SHAPES = [(1041, 3100, 128), (645, 5003, 256), (300, 9728, 384), (500, 4030, 896), (2090, 2601, 1024)]
+
+
+@pytest.mark.parametrize("m,n,k", SHAPES + [(200, 4100, 32), (777, 4096, 1056)])
+def test_mxfp4(rng, m, n, k):
+    W = lb.MXFP4Weights(rng.integers(0, 256, (n, k // 2), dtype=np.uint8),
+                        rng.integers(117, 131, (n, k // 32), dtype=np.uint8), k)
+    W.e8m0[0], W.e8m0[1] = 0, 254  # the smallest and the largest scale
+    W.e8m0[2, 0] = 255             # NaN
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    x[4] = 0
+    x[5] *= np.float32(2.0 ** 60)
+    x[6] *= np.float32(2.0 ** -90)
+    x[7, ::31] *= 4096             # large elements beside ordinary ones in every block
+    x[8, 1], x[9, 2] = np.inf, np.nan
+    y = K.gemm_mxfp4(x, lb.to_device(W))
+    assert np.isnan(y[8]).all() and np.isnan(y[9]).all() and np.isnan(y[:, 2]).all()
+    keep, cols = np.ones(m, bool), np.ones(n, bool)
+    keep[8:10], cols[:3] = False, False
+    ref = O.gemm_mxfp4_ref(x[keep], W.qw[cols], W.e8m0[cols])
+    bound = O.fp_bound(x[keep], O.dequant_mxfp4(W.qw[cols], W.e8m0[cols]))
+    O.assert_fp_close(y[np.ix_(keep, cols)], ref, bound, 1e-5)
+    assert np.array_equal(y[4, cols], np.zeros(cols.sum(), np.float32))
+
+
+def test_columns_that_take_nothing_from_huge_elements(rng):
+    """Where a row's few huge elements meet only zero weights, the other elements' products
+    must keep the bound, which the huge ones then add nothing to."""
+    m, n, k = 640, 4096, 512
+    huge = np.arange(7, k, 97)
+    codes = rng.integers(0, 16, (n, k), dtype=np.uint8)
+    codes[:, huge] = 0
+    W = lb.MXFP4Weights(lb.formats.pack_nibbles(codes, 32), rng.integers(122, 128, (n, k // 32), dtype=np.uint8), k)
+    D = lb.to_device(W)
+    for amp in (3e4, 3e9, 3e30):
+        x = rng.standard_normal((m, k)).astype(np.float32)
+        x[::2, huge] *= np.float32(amp)
+        O.assert_fp_close(K.gemm_mxfp4(x, D), O.gemm_mxfp4_ref(x, W.qw, W.e8m0), O.fp_bound(x, W.dequantize()), 1e-5)
