@@ -271,6 +271,7 @@ int run_bf3(int fmt, const lbk::GemmArgs &a0, char *ws, hipStream_t s, bool f8 =
   }
   if (e != hipSuccess) return fail_hip(e, "activation split launch");
   if (!prompt) e = lbk::launch_bf3_gemm(fmt, a, cus, s, f8);
+  else if (fmt == lbk::F_W4A16) e = lbk::launch_w4a16_prompt(a, tile, f8, s);
   else e = lbk::launch_mxfp4_prompt(a, tile, s);
   if (e != hipSuccess) return fail_hip(e, "bf16x3 GEMM launch");
   return ok(LB_ISA_GFX950_MFMA);

@@ -154,6 +154,8 @@ constexpr int kDigits = 7;
 size_t digit_bytes(int M, int Kp);
 hipError_t launch_split_digits(const float *x, int M, int Kp, void *out, hipStream_t s);
 hipError_t launch_mxfp4_prompt(const GemmArgs &a, PromptTile t, hipStream_t s);
+// W4A16 with many rows, on launch_split2h's activations and t16 or t16f8 (f8) weights.
+hipError_t launch_w4a16_prompt(const GemmArgs &a, PromptTile t, bool f8, hipStream_t s);
 // fp32 MFMA W4A16 / MXFP4.
 hipError_t launch_f32_mfma(int fmt, const GemmArgs &a, hipStream_t s);
 // exact int32 group accumulators through the VALU dot4 arithmetic of the GEMV.

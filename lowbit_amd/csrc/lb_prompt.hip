@@ -322,6 +322,171 @@ hipError_t launch_mxfp4_prompt(const GemmArgs &a, PromptTile t, hipStream_t s) {
   return launch_prompt(mxfp4_prompt_kernel<2, 4>, a, t, s);
 }
 
+// ============================================================ W4A16
+//
+// The arithmetic of the batch kernel (bf3_gemm_kernel with H2): two float16 terms per
+// activation, hi + lo 2^-11, each row times 2^xexp, against the exact float16 q - z; the
+// two sums of a group meet and take the group scale in float32, and eight groups' sums
+// meet before they join the total, so that the float32 roundings of a long K do not all
+// happen at the total's size.
+//
+//   t16 decode: the bytes 00 64 with the low one a nibble are the float16 1024 + q, less
+//   1024 + z exact. t16f8 weights, two conversions a dword, become the same operands in the
+//   same order, so both layouts give the same bits.
+template <int TM, int WN, bool F8>
+__global__ __launch_bounds__(kPThreads, 2) void w4a16_prompt_kernel(GemmArgs a, int mt, int nt) {
+  constexpr int SK = TM * 8, PW = SK / kPWaves;  // KiB of a stage, and of a wave's share
+  __shared__ __align__(16) char xs0[SK * 1024], xs1[SK * 1024];
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int q = lane >> 4, c = lane & 15;
+  const int M = a.M, N = a.N, Kp = a.Kp, G = Kp / kGroup, G4 = t16_groups(Kp), S = (N + 15) / 16;
+  int tm, tn;
+  if (!prompt_tile(mt, nt, tm, tn)) return;
+  const int mb0 = tm * TM, s0 = (tn * kPWaves + wave) * WN;
+  const Rsrc rx = make_rsrc(a.x3, (uint32_t)min(x2h_bytes(M, Kp), (size_t)0xFFFFFFF0u));
+  const Rsrc rw = make_rsrc(a.qw, (uint32_t)min(F8 ? t16f8_qw_bytes(N, Kp) : t16_qw_bytes(N, Kp), (size_t)0xFFFFFFF0u));
+  const size_t gents = t16_group_entries(N, Kp);
+  const Rsrc rs = make_rsrc(a.scales, (uint32_t)(gents * 4));
+  const Rsrc rz = make_rsrc(a.zeros ? a.zeros : a.qw, !F8 && a.zeros ? (uint32_t)gents : 0u);
+  const uint32_t zadd = a.zeros ? 0u : 8u;
+
+  struct Weights {
+    uint4 w[WN], w2[F8 ? WN : 1];
+    float s[WN];
+    uint32_t z[WN];
+  } wt;
+  constexpr int OPS = PW + 3 * WN;
+  const auto load = [&](int op, char *xd, int g) {
+    if (op < PW) {
+      const int t = wave * PW + op;  // KiB t % 8 of row block t / 8; past the last row block zeros
+      lds_load16(rx, xd + t * 1024, (((uint32_t)(mb0 + (t >> 3)) * G + g) * 8u + (t & 7)) * 1024u + (uint32_t)lane * 16u, 0);
+    } else if (op < OPS) {
+      const int j = (op - PW) / 3;
+      const uint32_t sj = (uint32_t)min(s0 + j, S - 1), gu = (sj * (G4 / 4) + g / 4) * 64u;
+      const uint32_t wb = (sj * G4 + g) * (F8 ? 2048u : 1024u);
+      if ((op - PW) % 3 == 0) wt.w[j] = ld_b128(rw, (uint32_t)lane * 16u, wb);
+      else if ((op - PW) % 3 == 1) wt.s[j] = ld_f32(rs, (uint32_t)c * 16u, (gu + (g & 3)) * 4u);
+      else if constexpr (F8) wt.w2[j] = ld_b128(rw, (uint32_t)lane * 16u, wb + 1024u);
+      else wt.z[j] = ld_u32(rz, (uint32_t)c * 4u, gu);
+    }
+  };
+  v4f facc[TM][WN], total[TM][WN];
+#pragma unroll
+  for (int i = 0; i < TM; i++)
+#pragma unroll
+    for (int j = 0; j < WN; j++) facc[i][j] = v4f{0.f, 0.f, 0.f, 0.f}, total[i][j] = facc[i][j];
+
+  const auto group = [&](const char *xd, char *nxd, int g) {
+    const int gn = min(g + 1, G - 1);
+    v4u b[WN][4];
+    float s[WN];
+#pragma unroll
+    for (int j = 0; j < WN; j++) {
+      s[j] = wt.s[j];
+      if constexpr (F8) {  // operand u, element e = lane byte 8 u + e, already less its zero-point
+        const uint32_t w[8] = {wt.w[j].x, wt.w[j].y, wt.w[j].z, wt.w[j].w, wt.w2[j].x, wt.w2[j].y, wt.w2[j].z, wt.w2[j].w};
+#pragma unroll
+        for (int d = 0; d < 8; d++) {
+          b[j][d >> 1][2 * (d & 1)] =
+              __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w[d], 512.0f, false));
+          b[j][d >> 1][2 * (d & 1) + 1] =
+              __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w[d], 512.0f, true));
+        }
+      } else {
+        const float z = (float)(((wt.z[j] >> (8 * (g & 3))) & 0xFFu) + zadd);
+        const h2v z2 = {(_Float16)(1024.0f + z), (_Float16)(1024.0f + z)};
+        const uint32_t w[4] = {wt.w[j].x, wt.w[j].y, wt.w[j].z, wt.w[j].w};
+#pragma unroll
+        for (int d = 0; d < 8; d++) {  // operands u = d / 2: low nibbles of dwords 0 .. 3, then high
+          const uint32_t nib = d < 4 ? lo_nibbles(w[d & 3]) : hi_nibbles(w[d & 3]);
+          const h2v lo = __builtin_bit_cast(h2v, __builtin_amdgcn_perm(0x64646464u, nib, 0x07010700u));
+          const h2v hi = __builtin_bit_cast(h2v, __builtin_amdgcn_perm(0x64646464u, nib, 0x07030702u));
+          b[j][d >> 1][2 * (d & 1)] = __builtin_bit_cast(uint32_t, lo - z2);
+          b[j][d >> 1][2 * (d & 1) + 1] = __builtin_bit_cast(uint32_t, hi - z2);
+        }
+      }
+    }
+    v8h xa[2][2];  // [parity][hi, lo] of step k = (row block k / 4, u = k % 4)
+    v4f dh[2][WN], dl[2][WN];
+    const auto read = [&](int k, int p) {
+      xa[k & 1][p] = *reinterpret_cast<const v8h *>(xd + (k * 2 + p) * 1024 + lane * 16);
+    };
+    // products of row block i go through the scale while row block i + 1 multiplies: merges
+    // first, then the scale (a dependent pair back to back stalls)
+    const auto scale = [&](int i, int slot) {
+      const int e0 = (slot % (2 * WN)) * 2;
+#pragma unroll
+      for (int e = e0; e < e0 + 2; e++) {
+        const int j = e >> 2, r = e & 3;
+        if (slot < 2 * WN) dh[i & 1][j][r] = __builtin_fmaf(dl[i & 1][j][r], 0x1p-11f, dh[i & 1][j][r]);
+        else facc[i][j][r] = __builtin_fmaf(s[j], dh[i & 1][j][r], facc[i][j][r]);
+      }
+    };
+    read(0, 0);
+    read(0, 1);
+    __builtin_amdgcn_sched_barrier(0);
+    int op = 0;
+#pragma unroll
+    for (int k = 0; k < 4 * TM; k++) {
+      const int i = k >> 2, u = k & 3;
+#pragma unroll
+      for (int j = 0; j < WN; j++) {
+        const v4f zero = {0.f, 0.f, 0.f, 0.f};
+        const v8h bj = __builtin_bit_cast(v8h, b[j][u]);
+        dh[i & 1][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[k & 1][0], bj, u ? dh[i & 1][j] : zero, 0, 0, 0);
+        if (j < 2 && k + 1 < 4 * TM) read(k + 1, j);
+        else load(op++, nxd, gn);
+        dl[i & 1][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[k & 1][1], bj, u ? dl[i & 1][j] : zero, 0, 0, 0);
+        if (i > 0) scale(i - 1, u * WN + j);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    static_assert((4 * TM - 1) * (WN - 2) + WN >= OPS, "every load has a slot");
+#pragma unroll
+    for (int n = 0; n < 4 * WN; n++) scale(TM - 1, n);
+  };
+  const auto meet = [&]() {
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+      for (int j = 0; j < WN; j++) total[i][j] += facc[i][j], facc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
+  };
+#pragma unroll
+  for (int op = 0; op < OPS; op++) load(op, xs0, 0);
+  const auto step = [&](const char *xd, char *nxd, int g) {
+    stage_ready<0>();
+    group(xd, nxd, g);
+  };
+  for (int g = 0; g < G; g += 2) {
+    step(xs0, xs1, g);
+    if (g + 1 < G) step(xs1, xs0, g + 1);
+    if ((g & 7) == 6) meet();
+  }
+  meet();
+  stage_ready<0>();  // no load to LDS outlives the workgroup
+#pragma unroll
+  for (int i = 0; i < TM; i++) {
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int m = (mb0 + i) * 16 + 4 * q + r;
+      if (m >= M) continue;
+      const int e = -a.xexp[m];
+#pragma unroll
+      for (int j = 0; j < WN; j++) {
+        const int n = 16 * (s0 + j) + c;
+        if (n < N) a.y[(size_t)m * N + n] = ldexpf(total[i][j][r], e);
+      }
+    }
+  }
+}
+
+hipError_t launch_w4a16_prompt(const GemmArgs &a, PromptTile t, bool f8, hipStream_t s) {
+  if (!a.wt16 || !a.x3 || !a.xexp) return hipErrorInvalidValue;
+  return f8 ? launch_prompt(w4a16_prompt_kernel<2, 4, true>, a, t, s)
+            : launch_prompt(w4a16_prompt_kernel<2, 4, false>, a, t, s);
+}
+
 // ============================================================ dispatch
 //
 // Where these kernels beat the batch kernels, from both sides' times (us) at 56 shapes of
@@ -333,6 +498,9 @@ hipError_t launch_mxfp4_prompt(const GemmArgs &a, PromptTile t, hipStream_t s) {
 //          CUs (256 x 4096 x 4096 29.5 -> 26.0). Wins from T = 12 at every K
 //          (192 x 4096 x 4096 38.8 -> 25.9, x 11008 87.8 -> 56.2, 1024 x 4096 x 4096 179 ->
 //          61; 128 rows 19.5 against 25.0, not taken).
+//   W4A16  1.13 us a group and round of 256 workgroups against 0.055 T of the batch kernel
+//          (512 x 4096 x 4096 60.5 -> 49.0, 2048 x 11008 x 4096 642 -> 364; 256 x 4096 x
+//          4096 39.9 against 44.4, not taken).
 // Few rows (32 and less) stay with the batch kernels, which are built for them.
 bool prompt_tile_for(int fmt, int M, int N, [[maybe_unused]] int Kp, int num_cus, PromptTile *out) {
   if (M <= 32) return false;
@@ -345,6 +513,9 @@ bool prompt_tile_for(int fmt, int M, int N, [[maybe_unused]] int Kp, int num_cus
   if (fmt == F_MXFP4) {
     if (T < 12) return false;
     t = PromptTile{rounds(1, 4) <= 1 ? 1 : 2, 4};
+  } else if (fmt == F_W4A16) {
+    t = PromptTile{2, 4};
+    if (1.13 * std::ceil(rounds(2, 4)) > 0.055 * T) return false;
   } else {
     return false;
   }

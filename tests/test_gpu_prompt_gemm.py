@@ -2,18 +2,49 @@
 subtiles past the matrix, one and an odd number of K groups, the stage buffers with every
 number of groups left over, the largest zero-points, against the float64 oracle within the
 bounds that the batch kernels' tests use."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
 import lowbit_amd as lb
 from lowbit_amd import kernels as K
 from oracle import reference as O
+from problems import outlier_int4_problem
 
 pytestmark = pytest.mark.gpu
 
 # M, N, K: ragged M and N, 1, 2, 3, 7 and 8 groups; 13 or more 16 x 16 tiles of Y per CU,
 # where every format takes these kernels
 SHAPES = [(1041, 3100, 128), (645, 5003, 256), (300, 9728, 384), (500, 4030, 896), (2090, 2601, 1024)]
+
+
+def _int4(rng, n, k, asym, zmax=15):
+    g = k // 128
+    return lb.Int4Weights(rng.integers(0, 256, (n, k // 2), dtype=np.uint8),
+                          (rng.standard_normal((n, g)) * 0.05).astype(np.float32),
+                          rng.integers(0, zmax + 1, (n, g), dtype=np.uint8) if asym else None, k)
+
+
+@pytest.mark.parametrize("m,n,k", SHAPES)
+@pytest.mark.parametrize("asym,zmax", [(False, 0), (True, 15), (True, 255)])
+def test_w4a16(rng, m, n, k, asym, zmax):
+    """Zero-points past 15 rule the t16f8 copy out; elsewhere it gives t16's bits."""
+    W = _int4(rng, n, k, asym, zmax)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    x[5] *= 1e30
+    x[6] *= 1e-30
+    D = lb.to_device(W)
+    y = K.gemm_w4a16(x, D)
+    O.assert_fp_close(y, O.gemm_w4a16_ref(x, W.qw, W.scales, W.zeros), O.fp_bound(x, W.dequantize()), 1e-5)
+    assert D.f8_exact() == (zmax <= 15)
+    if D.f8_exact():
+        qwt8, st = D.tiles_f8()
+        L, prm = K.lib(), K._Params(-1, 0, 0, 0, 0, 0, 0)
+        dx, dy = K.DeviceBuffer.from_array(x), K.DeviceBuffer(m * n * 4)
+        assert L.lbd_gemm_w4a16_t16f8(dx.ptr, m, k, qwt8.ptr, st.ptr, n, dy.ptr, C.byref(prm), None, 0,
+                                      None) == K.ISA_GFX950_MFMA
+        np.testing.assert_array_equal(dy.to_array((m, n), np.float32), y)
 
 
 @pytest.mark.parametrize("m,n,k", SHAPES + [(200, 4100, 32), (777, 4096, 1056)])
@@ -42,6 +73,9 @@ def test_columns_that_take_nothing_from_huge_elements(rng):
     """Where a row's few huge elements meet only zero weights, the other elements' products
     must keep the bound, which the huge ones then add nothing to."""
     m, n, k = 640, 4096, 512
+    x, W = outlier_int4_problem(rng, m, n, k)
+    O.assert_fp_close(K.gemm_w4a16(x, lb.to_device(W)), O.gemm_w4a16_ref(x, W.qw, W.scales, W.zeros),
+                      O.fp_bound(x, W.dequantize()), 1e-5)
     huge = np.arange(7, k, 97)
     codes = rng.integers(0, 16, (n, k), dtype=np.uint8)
     codes[:, huge] = 0
