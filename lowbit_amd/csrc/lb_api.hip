@@ -326,13 +326,15 @@ int run_w4a8(const lbk::GemmArgs &a, const lb_params *p, char *ws, hipStream_t s
   int8_t *xq = reinterpret_cast<int8_t *>(ws);
   float *xs = reinterpret_cast<float *>(ws + xq_bytes);
   int32_t *asum = reinterpret_cast<int32_t *>(ws + xq_bytes + align256((size_t)a.M * 4));
-  hipError_t e = lbk::launch_quant(a.x, a.M, a.Kp, xq, xs, asum, true, s);
+  lbk::PromptTile tile;
+  const bool prompt = a.wt16 && lbk::prompt_tile_for(lbk::F_W4A8, a.M, a.N, a.Kp, cus, &tile);
+  hipError_t e = lbk::launch_quant(a.x, a.M, a.Kp, xq, xs, asum, true, prompt, s);
   if (e != hipSuccess) return fail_hip(e, "quantizer launch");
   q.xq = xq;
   q.xs = xs;
   q.asum = asum;
   q.tiled = true;
-  e = lbk::launch_w4a8_mfma(q, nullptr, cus, s);
+  e = prompt ? lbk::launch_w4a8_prompt(q, tile, s) : lbk::launch_w4a8_mfma(q, nullptr, cus, s);
   if (e != hipSuccess) return fail_hip(e, "W4A8 MFMA launch");
   return ok(path);
 }
@@ -731,7 +733,7 @@ int lbd_quant_act_int8(const float *x, int M, int Kp, int8_t *xq, float *xs, int
   if (M <= 0 || Kp <= 0 || Kp % LB_GROUP) return fail(LB_ERR_SHAPE, "bad shape");
   if (!x || !xq || !xs || !asum) return fail(LB_ERR_ARG, "null pointer");
   if (!aligned16(x) || !aligned16(xq)) return fail(LB_ERR_ARG, "x and xq must be 16-byte aligned");
-  hipError_t e = lbk::launch_quant(x, M, Kp, xq, xs, asum, false, static_cast<hipStream_t>(stream));
+  hipError_t e = lbk::launch_quant(x, M, Kp, xq, xs, asum, false, false, static_cast<hipStream_t>(stream));
   if (e != hipSuccess) return fail_hip(e, "quantizer launch");
   return ok(0);
 }

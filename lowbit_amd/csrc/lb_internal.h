@@ -133,8 +133,10 @@ int gemv_wg_per_cu(const void *kern, size_t lds, int threads = 512);
 // the group-32 instantiations of the small-M kernels (lb_gemv_g32.hip)
 hipError_t launch_gemv_g32(int fmt, const GemmArgs &a, int num_cus, size_t lds, hipStream_t s, GemvPlan *plan);
 // Per-token int8 quantizer: xq, xs, asum as lb_quant_act_int8, or (tiled) xq and asum
-// in the MFMA path's tiled layout over ceil(M/16)*16 rows, padding rows zero.
-hipError_t launch_quant(const float *x, int M, int Kp, int8_t *xq, float *xs, int32_t *asum, bool tiled,
+// in the MFMA path's tiled layout over ceil(M/16)*16 rows, padding rows zero; (tiled and
+// magic) the sums as kPromptMagic - 64 asum, the C operands of the prompt GEMM.
+constexpr int kPromptMagic = 0x4B400000;  // bits of 1.5 * 2^23: + n is the float 12582912 + n, |n| < 2^22
+hipError_t launch_quant(const float *x, int M, int Kp, int8_t *xq, float *xs, int32_t *asum, bool tiled, bool magic,
                         hipStream_t s);
 // Bytes of the tiled xq / asum for M rows.
 inline size_t tiled_xq_bytes(int M, int Kp) { return (size_t)((M + 15) / 16) * 16 * Kp; }
@@ -148,6 +150,9 @@ struct PromptTile {
 };
 // Whether a t16 GEMM of this shape runs faster on them than on the batch kernels, and how.
 bool prompt_tile_for(int fmt, int M, int N, int Kp, int num_cus, PromptTile *out);
+// W4A8 with many rows (lb_prompt.hip) on t16 weights and the quantizer's tiled (magic)
+// activations.
+hipError_t launch_w4a8_prompt(const GemmArgs &a, PromptTile t, hipStream_t s);
 // MXFP4 with many rows (lb_prompt.hip): the activations as kDigits E2M3 digits per
 // element (digit_bytes(M, Kp) bytes, within x3_bytes), the GEMM on them and t16 weights.
 constexpr int kDigits = 7;

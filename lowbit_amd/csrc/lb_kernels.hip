@@ -60,8 +60,9 @@ __device__ __forceinline__ uint32_t w4a8_tiled_offset(int m, int e, int G) {
 // (offsets past the row read 0), so all loads are in flight together; NR == 0
 // streams longer rows twice. The absmax is reduced across the workgroup and each
 // thread quantizes its 4-element slots with the exact fast path; group sums land
-// in asum.
-template <int NR, bool TILED>
+// in asum; for the prompt GEMM (MAGIC) as kPromptMagic - 64 times the sum, the C
+// operand it starts its integer products from.
+template <int NR, bool TILED, bool MAGIC>
 __global__ __launch_bounds__(kThreads) void quant_rows_kernel(
     const float *__restrict__ x, int M, int Kp, int8_t *__restrict__ xq, float *__restrict__ xs,
     int32_t *__restrict__ asum) {
@@ -72,7 +73,8 @@ __global__ __launch_bounds__(kThreads) void quant_rows_kernel(
     // padding rows of the last 16-row block: zero codes and sums
     for (int e = threadIdx.x * 4; e < Kp; e += kThreads * 4)
       *reinterpret_cast<uint32_t *>(xq + w4a8_tiled_offset(m, e, G)) = 0u;
-    for (int g = threadIdx.x; g < G; g += kThreads) asum[((m >> 4) * G + g) * 16 + (m & 15)] = 0;
+    for (int g = threadIdx.x; g < G; g += kThreads)
+      asum[((m >> 4) * G + g) * 16 + (m & 15)] = MAGIC ? kPromptMagic : 0;
     return;
   }
   const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
@@ -110,7 +112,7 @@ __global__ __launch_bounds__(kThreads) void quant_rows_kernel(
     const int gs = half_wave_sum(sum_i8x4(qv));
     if constexpr (TILED) {
       *reinterpret_cast<uint32_t *>(xq + w4a8_tiled_offset(m, e, G)) = qv;
-      if ((threadIdx.x & 31) == 31) asum[((m >> 4) * G + (e >> 7)) * 16 + (m & 15)] = gs;
+      if ((threadIdx.x & 31) == 31) asum[((m >> 4) * G + (e >> 7)) * 16 + (m & 15)] = MAGIC ? kPromptMagic - 64 * gs : gs;
     } else {
       reinterpret_cast<uint32_t *>(xq + (size_t)m * Kp)[e >> 2] = qv;
       if ((threadIdx.x & 31) == 31) asum[(size_t)m * G + (e >> 7)] = gs;
@@ -171,30 +173,24 @@ hipError_t launch_gemv(int fmt, const GemmArgs &a, int num_cus, hipStream_t s, G
   return hipErrorInvalidValue;
 }
 
-template <bool TILED>
+template <bool TILED, bool MAGIC>
 static void launch_quant_t(const float *x, int M, int Kp, int8_t *xq, float *xs, int32_t *asum, hipStream_t s) {
   const int n4 = (Kp + kThreads * 4 - 1) / (kThreads * 4);  // 16-byte slots per thread
   const dim3 grid(TILED ? (M + 15) / 16 * 16 : M), block(kThreads);
-  if (n4 <= 1)
-    hipLaunchKernelGGL((quant_rows_kernel<1, TILED>), grid, block, 0, s, x, M, Kp, xq, xs, asum);
-  else if (n4 <= 2)
-    hipLaunchKernelGGL((quant_rows_kernel<2, TILED>), grid, block, 0, s, x, M, Kp, xq, xs, asum);
-  else if (n4 <= 4)
-    hipLaunchKernelGGL((quant_rows_kernel<4, TILED>), grid, block, 0, s, x, M, Kp, xq, xs, asum);
-  else if (n4 <= 8)
-    hipLaunchKernelGGL((quant_rows_kernel<8, TILED>), grid, block, 0, s, x, M, Kp, xq, xs, asum);
-  else if (n4 <= 16)
-    hipLaunchKernelGGL((quant_rows_kernel<16, TILED>), grid, block, 0, s, x, M, Kp, xq, xs, asum);
-  else
-    hipLaunchKernelGGL((quant_rows_kernel<0, TILED>), grid, block, 0, s, x, M, Kp, xq, xs, asum);
+  auto go = [&](auto kern) { hipLaunchKernelGGL(kern, grid, block, 0, s, x, M, Kp, xq, xs, asum); };
+  if (n4 <= 1) go(quant_rows_kernel<1, TILED, MAGIC>);
+  else if (n4 <= 2) go(quant_rows_kernel<2, TILED, MAGIC>);
+  else if (n4 <= 4) go(quant_rows_kernel<4, TILED, MAGIC>);
+  else if (n4 <= 8) go(quant_rows_kernel<8, TILED, MAGIC>);
+  else if (n4 <= 16) go(quant_rows_kernel<16, TILED, MAGIC>);
+  else go(quant_rows_kernel<0, TILED, MAGIC>);
 }
 
-hipError_t launch_quant(const float *x, int M, int Kp, int8_t *xq, float *xs, int32_t *asum, bool tiled,
+hipError_t launch_quant(const float *x, int M, int Kp, int8_t *xq, float *xs, int32_t *asum, bool tiled, bool magic,
                         hipStream_t s) {
-  if (tiled)
-    launch_quant_t<true>(x, M, Kp, xq, xs, asum, s);
-  else
-    launch_quant_t<false>(x, M, Kp, xq, xs, asum, s);
+  if (tiled && magic) launch_quant_t<true, true>(x, M, Kp, xq, xs, asum, s);
+  else if (tiled) launch_quant_t<true, false>(x, M, Kp, xq, xs, asum, s);
+  else launch_quant_t<false, false>(x, M, Kp, xq, xs, asum, s);
   return hipGetLastError();
 }
 

@@ -66,6 +66,183 @@ static hipError_t launch_prompt(Kern kern, const GemmArgs &a, PromptTile t, hipS
   return hipGetLastError();
 }
 
+// ============================================================ W4A8
+//
+// The exact int32 group accumulators come out of the int8 MFMAs as float bits: the
+// first product's C operand is the bit pattern of 1.5 * 2^23 (whose unit is 1), so the
+// accumulator 1.5 * 2^23 + sum, |sum| < 2^18, is that float's bit pattern plus an
+// integer, i.e. the float 12582912 + sum exactly. One subtraction (a full-rate
+// instruction, unlike an int conversion) and one FMA with the group scale per output.
+// Codes enter as q - z + 64 (a positive byte for z <= 64: no borrow between bytes); the
+// activations' group sums, times -64, are part of the C operand (kPromptMagic - 64 asum,
+// which the quantizer writes in place of the sums). Zero-points above 64, which no
+// packer writes, are taken off afterwards, in float, as in the batch kernel.
+template <int TM, int WN>
+__global__ __launch_bounds__(kPThreads, 2) void w4a8_prompt_kernel(GemmArgs a, int mt, int nt) {
+  constexpr int SA = TM * 2048;  // bytes of a stage's operand tiles
+  __shared__ __align__(16) char xs0[SA], xs1[SA];
+  constexpr int CW = (TM + 3) / 4;  // loads of 4 row blocks' C values
+  __shared__ __align__(16) char cs0[CW * 256], cs1[CW * 256];
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int q = lane >> 4, c = lane & 15;
+  const int M = a.M, N = a.N, Kp = a.Kp, G = Kp / kGroup, G4 = t16_groups(Kp), S = (N + 15) / 16;
+  int tm, tn;
+  if (!prompt_tile(mt, nt, tm, tn)) return;
+  const int mb0 = tm * TM, s0 = (tn * kPWaves + wave) * WN;
+  const uint32_t mblocks = (uint32_t)((M + 15) / 16);
+  const Rsrc rx = make_rsrc(a.xq, mblocks * 16u * (uint32_t)Kp);
+  const Rsrc rc = make_rsrc(a.asum, mblocks * (uint32_t)G * 64u);
+  const Rsrc rw = make_rsrc(a.qw, (uint32_t)min(t16_qw_bytes(N, Kp), (size_t)0xFFFFFFF0u));
+  const size_t gents = t16_group_entries(N, Kp);
+  const Rsrc rs = make_rsrc(a.scales, (uint32_t)(gents * 4));
+  const Rsrc rz = make_rsrc(a.zeros ? a.zeros : a.qw, a.zeros ? (uint32_t)gents : 0u);
+  const uint32_t zadd = a.zeros ? 0u : 8u;
+
+  // stage of group g: row block i's two operand tiles (2 KiB, consecutive) and its 16 C values;
+  // row blocks past the last read 0
+  const auto stage = [&](char *xd, char *cd, int g) {
+#pragma unroll
+    for (int k = 0; k < TM * 2 / kPWaves; k++) {
+      const int t = wave * (TM * 2 / kPWaves) + k, i = t >> 1, h = t & 1;
+      lds_load16(rx, xd + t * 1024, ((((uint32_t)(mb0 + i) * G + g) * 2 + h) * kWave + lane) * 16u, 0);
+    }
+    // every wave loads (the same values where there are fewer loads than waves): a load that
+    // only some paths issue would make the waits below count on it never having been issued
+    const int cw = wave % CW;
+    lds_load4(rc, cd + cw * 256, (((uint32_t)(mb0 + 4 * cw + q) * G + g) * 16 + c) * 4u, 0);
+  };
+  struct Weights {
+    uint4 w[WN];
+    float s[WN];
+    uint32_t z[WN];
+  } w0, w1;
+  // subtiles past the last one read it again (their columns are not stored)
+  const auto weights = [&](Weights &n, int g) {
+#pragma unroll
+    for (int j = 0; j < WN; j++) {
+      const uint32_t sj = (uint32_t)min(s0 + j, S - 1);
+      n.w[j] = ld_b128(rw, (uint32_t)lane * 16u, (sj * G4 + g) * 1024u);
+      const uint32_t gu = (sj * (G4 / 4) + g / 4) * 64u;
+      n.s[j] = ld_f32(rs, (uint32_t)c * 16u, (gu + (g & 3)) * 4u);
+      n.z[j] = ld_u32(rz, (uint32_t)c * 4u, gu);  // no zero-points: a zero-length range reads 0
+    }
+  };
+  v4f facc[TM][WN];
+#pragma unroll
+  for (int i = 0; i < TM; i++)
+#pragma unroll
+    for (int j = 0; j < WN; j++) facc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
+
+  const auto group = [&](const char *xd, const char *cd, const Weights &n, int g) {
+    v4i blo[WN], bhi[WN];
+    float s[WN];
+    int rz4[WN], over = 0;
+#pragma unroll
+    for (int j = 0; j < WN; j++) {
+      s[j] = n.s[j];
+      const uint32_t z = ((n.z[j] >> (8 * (g & 3))) & 0xFFu) + zadd, z64 = min(z, 64u);
+      rz4[j] = (int)(z - z64);
+      over |= rz4[j];
+      const uint32_t add = 0x40404040u - __builtin_amdgcn_perm(z64, z64, 0u);
+      const uint32_t w[4] = {n.w[j].x, n.w[j].y, n.w[j].z, n.w[j].w};
+#pragma unroll
+      for (int d = 0; d < 4; d++) {
+        blo[j][d] = (int)(lo_nibbles(w[d]) + add);
+        bhi[j][d] = (int)(hi_nibbles(w[d]) + add);
+      }
+    }
+    // row block i's operands are read while block i - 1 multiplies, and its products are
+    // scaled while block i + 1 does
+    v4i xlo[2], xhi[2], ci[2], acc[2][WN];
+    const auto read = [&](int i) {
+      xlo[i & 1] = *reinterpret_cast<const v4i *>(xd + (2 * i) * 1024 + lane * 16);
+      xhi[i & 1] = *reinterpret_cast<const v4i *>(xd + (2 * i + 1) * 1024 + lane * 16);
+      ci[i & 1] = *reinterpret_cast<const v4i *>(cd + i * 64 + q * 16);
+    };
+    // (subtractions and FMAs in phases of their own: a dependent pair back to back stalls)
+    const auto unbias = [&](int i) {
+#pragma unroll
+      for (int j = 0; j < WN; j++)
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+          acc[i & 1][j][r] = __float_as_int(__int_as_float(acc[i & 1][j][r]) - 12582912.0f);
+    };
+    const auto scale = [&](int i) {
+#pragma unroll
+      for (int j = 0; j < WN; j++)
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+          facc[i][j][r] = __builtin_fmaf(__int_as_float(acc[i & 1][j][r]), s[j], facc[i][j][r]);
+    };
+    read(0);
+#pragma unroll
+    for (int i = 0; i < TM; i++) {
+      const int b = i & 1;
+      if (i + 1 < TM) read(i + 1);
+#pragma unroll
+      for (int j = 0; j < WN; j++) acc[b][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(xlo[b], blo[j], ci[b], 0, 0, 0);
+      if (i > 0) unbias(i - 1);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int j = 0; j < WN; j++)
+        acc[b][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(xhi[b], bhi[j], acc[b][j], 0, 0, 0);
+      if (i > 0) scale(i - 1);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    unbias(TM - 1);
+    __builtin_amdgcn_sched_barrier(0);
+    scale(TM - 1);
+    if (__any(over)) {
+#pragma unroll
+      for (int i = 0; i < TM; i++) {
+        const v4i ci = *reinterpret_cast<const v4i *>(cd + i * 64 + q * 16);
+#pragma unroll
+        for (int j = 0; j < WN; j++)
+#pragma unroll
+          for (int r = 0; r < 4; r++)
+            facc[i][j][r] = __builtin_fmaf((float)(rz4[j] * ((ci[r] - kPromptMagic) >> 6)), s[j], facc[i][j][r]);
+      }
+    }
+  };
+  stage(xs0, cs0, 0);
+  weights(w0, 0);
+  // the next group's loads are issued first (the scheduler would sink them to the end)
+  const auto step = [&](char *xd, char *cd, Weights &n, char *nxd, char *ncd, Weights &nn, int g) {
+    stage_ready<0>();
+    stage(nxd, ncd, min(g + 1, G - 1));
+    weights(nn, min(g + 1, G - 1));
+    __builtin_amdgcn_sched_barrier(0);
+    group(xd, cd, n, g);
+  };
+  for (int g = 0; g < G; g += 2) {
+    step(xs0, cs0, w0, xs1, cs1, w1, g);
+    if (g + 1 < G) step(xs1, cs1, w1, xs0, cs0, w0, g + 1);
+  }
+  stage_ready<0>();  // no load to LDS outlives the workgroup
+#pragma unroll
+  for (int i = 0; i < TM; i++) {
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int m = (mb0 + i) * 16 + 4 * q + r;
+      if (m >= M) continue;
+      const float xs = a.xs[m];
+#pragma unroll
+      for (int j = 0; j < WN; j++) {
+        const int n = 16 * (s0 + j) + c;
+        if (n < N) a.y[(size_t)m * N + n] = facc[i][j][r] * xs;
+      }
+    }
+  }
+}
+
+hipError_t launch_w4a8_prompt(const GemmArgs &a, PromptTile t, hipStream_t s) {
+  if (!a.wt16 || !a.tiled) return hipErrorInvalidValue;
+  if (t.tm == 8) return launch_prompt(w4a8_prompt_kernel<8, 2>, a, t, s);
+  if (t.tm == 4) return launch_prompt(w4a8_prompt_kernel<4, 2>, a, t, s);
+  return launch_prompt(w4a8_prompt_kernel<2, 2>, a, t, s);
+}
+
 // ============================================================ MXFP4
 //
 // The MX matrix instruction (v_mfma_scale_f32_16x16x128_f8f6f4) takes E2M1 weights and
@@ -501,10 +678,16 @@ hipError_t launch_w4a16_prompt(const GemmArgs &a, PromptTile t, bool f8, hipStre
 //   W4A16  1.13 us a group and round of 256 workgroups against 0.055 T of the batch kernel
 //          (512 x 4096 x 4096 60.5 -> 49.0, 2048 x 11008 x 4096 642 -> 364; 256 x 4096 x
 //          4096 39.9 against 44.4, not taken).
+//   W4A8   32-, 64- and 128-row tiles: 0.57, 0.72, 1.13 us a group, 0.0205, 0.0163, 0.0140 T
+//          when the chip is full, against 0.0235 T a group of the batch kernel, which
+//          works on phases of 32 groups (1024 x 4096 x 11008 231 -> 90, 384 x 4096 x 1024
+//          22.9 -> 12.4, 2048 x 11008 x 4096 252 -> 150; 256 x 4096 x 4096 17.8 against 25).
 // Few rows (32 and less) stay with the batch kernels, which are built for them.
-bool prompt_tile_for(int fmt, int M, int N, [[maybe_unused]] int Kp, int num_cus, PromptTile *out) {
+bool prompt_tile_for(int fmt, int M, int N, int Kp, int num_cus, PromptTile *out) {
   if (M <= 32) return false;
-  const double cus = num_cus > 0 ? num_cus : 256;
+  // 32-bit offsets, up to a tile past the last row (the other formats' callers have checked)
+  if (fmt == F_W4A8 && ((size_t)M + 160) * Kp > 0xFFFFFF00u) return false;
+  const double cus = num_cus > 0 ? num_cus : 256, G = (Kp + 127) / 128;
   const double T = (double)((M + 15) / 16) * ((N + 15) / 16) / cus;
   const auto rounds = [&](int tm, int wn) {
     return (double)((M + 16 * tm - 1) / (16 * tm)) * ((N + 64 * wn - 1) / (64 * wn)) / cus;
@@ -516,6 +699,11 @@ bool prompt_tile_for(int fmt, int M, int N, [[maybe_unused]] int Kp, int num_cus
   } else if (fmt == F_W4A16) {
     t = PromptTile{2, 4};
     if (1.13 * std::ceil(rounds(2, 4)) > 0.055 * T) return false;
+  } else if (fmt == F_W4A8) {
+    const double per[3] = {std::max(0.57, 0.0205 * T), std::max(0.72, 0.0163 * T), std::max(1.13, 0.0140 * T)};
+    const int best = (int)(std::min_element(per, per + 3) - per);
+    t = PromptTile{2 << best, 2};
+    if (1.0 + G * per[best] > 0.9 * 0.0235 * T * 32 * std::ceil(G / 32)) return false;
   } else {
     return false;
   }

@@ -9,6 +9,7 @@ import pytest
 
 import lowbit_amd as lb
 from lowbit_amd import kernels as K
+from oracle import cref
 from oracle import reference as O
 from problems import outlier_int4_problem
 
@@ -24,6 +25,19 @@ def _int4(rng, n, k, asym, zmax=15):
     return lb.Int4Weights(rng.integers(0, 256, (n, k // 2), dtype=np.uint8),
                           (rng.standard_normal((n, g)) * 0.05).astype(np.float32),
                           rng.integers(0, zmax + 1, (n, g), dtype=np.uint8) if asym else None, k)
+
+
+@pytest.mark.parametrize("m,n,k", SHAPES)
+@pytest.mark.parametrize("asym,zmax", [(False, 0), (True, 15), (True, 255)])
+def test_w4a8(rng, m, n, k, asym, zmax):
+    W = _int4(rng, n, k, asym, zmax)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    x[3] = 0
+    y = K.gemm_w4a8(x, lb.to_device(W))
+    a = lb.quantize_act_int8(x)
+    ref, bound = cref.c_gemm_w4a8(a.xq, a.scale, a.gsum, W.qw, W.scales, W.zeros)
+    O.assert_fp_close(y, ref, bound, 1e-5)
+    assert np.array_equal(y[3], np.zeros(n, np.float32))
 
 
 @pytest.mark.parametrize("m,n,k", SHAPES)
