@@ -55,6 +55,16 @@ __device__ __forceinline__ uint32_t w4a8_tiled_offset(int m, int e, int G) {
   return (uint32_t)((((((m >> 4) * G + g) * 2 + (r >> 6)) * 64 + ((r >> 4) & 3) * 16 + (m & 15)) * 16) + (r & 15));
 }
 //
+// Row of a workgroup that writes one row of 16-row operand tiles: workgroups go to the 8
+// XCDs in turn, so with a grid of whole 128s the 16 rows of a block, whose 4- and 16-byte
+// pieces share cache lines, are given to one XCD, whose L2 puts the lines together (whole
+// GEMMs: W4A16 512 x 4096 x 4096 48.9 -> 46.1 us, W4A8 1000 x 4096 x 11008 91.7 -> 84.6).
+// Up to 112 rows the grid stays exact, without the two instructions: too few lines for it to
+// matter (W4A8 64 x 11008 x 4096 12.14 against 12.24 us with it).
+constexpr int kRowsInTurn = 112;
+__device__ __forceinline__ int row_of_block(int b) { return (b & ~127) | ((b & 7) << 4) | ((b >> 3) & 15); }
+static unsigned row_grid(int M) { return (unsigned)((M + 127) / 128 * 128); }
+//
 // One workgroup per activation row. With NR > 0 the row (at most NR * 1024
 // elements) is loaded into registers by NR unconditional 16-byte loads per thread
 // (offsets past the row read 0), so all loads are in flight together; NR == 0
@@ -62,13 +72,14 @@ __device__ __forceinline__ uint32_t w4a8_tiled_offset(int m, int e, int G) {
 // thread quantizes its 4-element slots with the exact fast path; group sums land
 // in asum; for the prompt GEMM (MAGIC) as kPromptMagic - 64 times the sum, the C
 // operand it starts its integer products from.
-template <int NR, bool TILED, bool MAGIC>
+template <int NR, bool TILED, bool MAGIC, bool BYXCD>
 __global__ __launch_bounds__(kThreads) void quant_rows_kernel(
     const float *__restrict__ x, int M, int Kp, int8_t *__restrict__ xq, float *__restrict__ xs,
     int32_t *__restrict__ asum) {
   __shared__ float red[kWaves];
-  const int m = blockIdx.x;
+  const int m = BYXCD ? row_of_block(blockIdx.x) : blockIdx.x;
   const int G = Kp / kGroup;
+  if (BYXCD && m >= (M + 15) / 16 * 16) return;
   if (TILED && m >= M) {
     // padding rows of the last 16-row block: zero codes and sums
     for (int e = threadIdx.x * 4; e < Kp; e += kThreads * 4)
@@ -173,24 +184,25 @@ hipError_t launch_gemv(int fmt, const GemmArgs &a, int num_cus, hipStream_t s, G
   return hipErrorInvalidValue;
 }
 
-template <bool TILED, bool MAGIC>
+template <bool TILED, bool MAGIC, bool BYXCD>
 static void launch_quant_t(const float *x, int M, int Kp, int8_t *xq, float *xs, int32_t *asum, hipStream_t s) {
   const int n4 = (Kp + kThreads * 4 - 1) / (kThreads * 4);  // 16-byte slots per thread
-  const dim3 grid(TILED ? (M + 15) / 16 * 16 : M), block(kThreads);
+  const dim3 grid(BYXCD ? row_grid(M) : TILED ? (M + 15) / 16 * 16 : M), block(kThreads);
   auto go = [&](auto kern) { hipLaunchKernelGGL(kern, grid, block, 0, s, x, M, Kp, xq, xs, asum); };
-  if (n4 <= 1) go(quant_rows_kernel<1, TILED, MAGIC>);
-  else if (n4 <= 2) go(quant_rows_kernel<2, TILED, MAGIC>);
-  else if (n4 <= 4) go(quant_rows_kernel<4, TILED, MAGIC>);
-  else if (n4 <= 8) go(quant_rows_kernel<8, TILED, MAGIC>);
-  else if (n4 <= 16) go(quant_rows_kernel<16, TILED, MAGIC>);
-  else go(quant_rows_kernel<0, TILED, MAGIC>);
+  if (n4 <= 1) go(quant_rows_kernel<1, TILED, MAGIC, BYXCD>);
+  else if (n4 <= 2) go(quant_rows_kernel<2, TILED, MAGIC, BYXCD>);
+  else if (n4 <= 4) go(quant_rows_kernel<4, TILED, MAGIC, BYXCD>);
+  else if (n4 <= 8) go(quant_rows_kernel<8, TILED, MAGIC, BYXCD>);
+  else if (n4 <= 16) go(quant_rows_kernel<16, TILED, MAGIC, BYXCD>);
+  else go(quant_rows_kernel<0, TILED, MAGIC, BYXCD>);
 }
 
 hipError_t launch_quant(const float *x, int M, int Kp, int8_t *xq, float *xs, int32_t *asum, bool tiled, bool magic,
                         hipStream_t s) {
-  if (tiled && magic) launch_quant_t<true, true>(x, M, Kp, xq, xs, asum, s);
-  else if (tiled) launch_quant_t<true, false>(x, M, Kp, xq, xs, asum, s);
-  else launch_quant_t<false, false>(x, M, Kp, xq, xs, asum, s);
+  if (tiled && magic) launch_quant_t<true, true, true>(x, M, Kp, xq, xs, asum, s);
+  else if (tiled && M > kRowsInTurn) launch_quant_t<true, false, true>(x, M, Kp, xq, xs, asum, s);
+  else if (tiled) launch_quant_t<true, false, false>(x, M, Kp, xq, xs, asum, s);
+  else launch_quant_t<false, false, false>(x, M, Kp, xq, xs, asum, s);
   return hipGetLastError();
 }
 
@@ -947,10 +959,13 @@ hipError_t launch_split3(int fmt, const float *x, int M, int Kp, uint4 *x3, hipS
 // per slot.
 // Workgroups (m, p) of a row each take the row's maximum over all of it (from the
 // caches after the first) and split part p of its slots.
+template <bool BYXCD>
 __global__ __launch_bounds__(kThreads) void split2h_kernel(const float *__restrict__ x, int M, int Kp,
                                                           uint4 *__restrict__ x2, int *__restrict__ xexp) {
   __shared__ float red[kThreads / kWave];
-  const int m = blockIdx.x, G = Kp / 128, items = G * 16;  // (g, u, q): 8 elements each
+  const int m = BYXCD ? row_of_block(blockIdx.x) : blockIdx.x;
+  const int G = Kp / 128, items = G * 16;  // (g, u, q): 8 elements each
+  if (BYXCD && m >= M) return;
   const int P = gridDim.y, pt0 = (int)(((long long)items * blockIdx.y) / P),
             pt1 = (int)(((long long)items * (blockIdx.y + 1)) / P);
   const float *xr = x + (size_t)m * Kp;
@@ -1000,7 +1015,10 @@ hipError_t launch_split2h(const float *x, int M, int Kp, uint4 *x2, int *xexp, h
   if (M <= 0 || Kp % 128) return hipErrorInvalidValue;
   // about 256 workgroups: each row's slots in up to G parts
   const int G = Kp / 128, P = std::max(1, std::min(G, 256 / M));
-  hipLaunchKernelGGL(split2h_kernel, dim3(M, P), dim3(kThreads), 0, s, x, M, Kp, x2, xexp);
+  if (M > kRowsInTurn)
+    hipLaunchKernelGGL(split2h_kernel<true>, dim3(row_grid(M), P), dim3(kThreads), 0, s, x, M, Kp, x2, xexp);
+  else
+    hipLaunchKernelGGL(split2h_kernel<false>, dim3(M, P), dim3(kThreads), 0, s, x, M, Kp, x2, xexp);
   return hipGetLastError();
 }
 
