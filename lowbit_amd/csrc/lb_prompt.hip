@@ -466,8 +466,10 @@ __global__ __launch_bounds__(kPThreads, 2) void mxfp4_prompt_kernel(GemmArgs a, 
   // two groups are in flight ahead of the one that runs
 #pragma unroll
   for (int op = 0; op < OPS; op++) load(op, xs0, w0, 0);
+  __builtin_amdgcn_sched_barrier(0);  // stage_ready counts on all of group 0's loads coming first
 #pragma unroll
   for (int op = 0; op < OPS; op++) load(op, xs1, w1, min(1, G - 1));
+  __builtin_amdgcn_sched_barrier(0);
   const auto step = [&](const char *xd, const Weights &n, char *nxd, Weights &nn, int g) {
     stage_ready<OPS>();
     group(xd, n, nxd, nn, g);

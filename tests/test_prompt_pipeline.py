@@ -1,0 +1,59 @@
+"""The load pipeline of the MXFP4 prompt GEMM in the code the compiler makes of it (CPU
+only: it compiles lb_prompt.hip to gfx950 assembly).
+
+The kernel waits for a stage by count: "all of this wave's loads but the last OPS have
+arrived". That holds only if the loads of an earlier group are issued before every load of
+a later one, which the scheduler does not know. The loop's order is pinned slot by slot;
+the two groups loaded ahead of it must be apart too.
+"""
+import re
+import shutil
+import subprocess
+from pathlib import Path
+
+import pytest
+
+from lowbit_amd import _build
+
+ROOT = Path(__file__).resolve().parents[1]
+KERNEL = "mxfp4_prompt_kernel"
+
+
+def _hipcc():
+    p = Path("/opt/rocm/bin/hipcc")
+    return str(p) if p.exists() else shutil.which("hipcc")
+
+
+@pytest.fixture(scope="module")
+def kernels(tmp_path_factory):
+    """The kernel's instantiations, each as its instructions (the entry block first)."""
+    cc = _hipcc()
+    if cc is None:
+        pytest.skip("hipcc not available")
+    out = tmp_path_factory.mktemp("asm") / "lb_prompt.s"
+    flags = [f for f in _build.FLAGS if f != "-shared"]
+    subprocess.run([cc, "--offload-arch=gfx950", *flags, f"-I{_build.INCLUDE}", "--offload-device-only", "-S",
+                    str(_build.CSRC / "lb_prompt.hip"), "-o", str(out)], check=True, capture_output=True, text=True)
+    found, name = {}, None
+    for line in out.read_text().splitlines():
+        m = re.match(r"(_Z\w+):", line)
+        if m:
+            name = m.group(1)
+        elif line.startswith("\t.section") or line.startswith("\t.p2align"):
+            name = None
+        elif name and KERNEL in name:
+            found.setdefault(name, []).append(line.split(";")[0].strip())
+    assert len(found) == 2, list(found)
+    return found
+
+
+def test_groups_loaded_ahead_are_apart(kernels):
+    """Before the loop: the loads to LDS of group 0, its weights', then those of group 1."""
+    for name, code in kernels.items():
+        kinds = []
+        for ins in code[:next(i for i, s in enumerate(code) if s.startswith("s_barrier"))]:
+            if ins.startswith("buffer_load"):
+                kinds.append("lds" if ins.endswith("lds") else "weights")
+        runs = [k for i, k in enumerate(kinds) if i == 0 or kinds[i - 1] != k]
+        assert runs == ["lds", "weights", "lds", "weights"], (name, runs)
+        assert kinds[:len(kinds) // 2] == kinds[len(kinds) // 2:], (name, kinds)
