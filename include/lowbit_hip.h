@@ -231,10 +231,11 @@ size_t lbd_bf16x3_workspace_bytes(int M, int Kp);
  * activations, then the slices' partial outputs, added by one more launch in slice
  * order. A workspace of this size (or NULL) takes the split, one of
  * lbd_bf16x3_workspace_bytes the unsplit GEMM; both meet the same bound, not the
- * same bits. (Shapes of many rows that run as prompt GEMMs take no split and leave the
- * room for it unused.) Equals lbd_bf16x3_workspace_bytes rounded up to 256 where no
- * split is taken; 0 for an invalid argument. (No reference counterpart: the reference's
- * GEMMs take no workspace.) */
+ * same bits. (W4A16 shapes of many rows that run as prompt GEMMs take no split and leave
+ * the room for it unused.) MXFP4 shapes of many rows that run as prompt GEMMs with this
+ * size, and as the batch kernel with lbd_bf16x3_workspace_bytes, take 1/48 more than the
+ * latter. Elsewhere it equals lbd_bf16x3_workspace_bytes rounded up to 256; 0 for an
+ * invalid argument. (No reference counterpart: the reference's GEMMs take no workspace.) */
 size_t lbd_bf16x3_workspace_bytes_split(int kind, int M, int N, int Kp);
 /* ---- "t16f8": int4 g128 weights for lbd_gemm_w4a16 on the matrix cores with the
  *      zero-point folded in (no reference counterpart: a device-private copy of an
@@ -272,8 +273,9 @@ int lbd_repack_mxfp4_t16(const uint8_t *qw, const uint8_t *e8m0, int N, int Kp,
 /* y = x . w^T as lbd_gemm_mxfp4 on t16 weights, the bf16 matrix-core path of
  * lbd_gemm_w4a16_t16 (block scales 2^(e - 127) exact; E8M0 255 gives NaN). With many
  * rows it runs on the MX matrix instruction instead, which takes the weights as they
- * are: the activations become 7 six-bit digits per element (more beside an outlier that
- * they do not reach), within the same workspace. */
+ * are: blocks of 32 activations whose nonzero magnitudes lie within 2^17 of each other
+ * become 8 six-bit digits per element, which hold them exactly; other blocks go through
+ * the three bf16 terms. A workspace of lbd_bf16x3_workspace_bytes_split bytes, or NULL. */
 int lbd_gemm_mxfp4_t16(const float *x, int M, int Kp, const uint8_t *qwt,
                        const uint8_t *et, int N, float *y, const lb_params *p,
                        void *workspace, size_t workspace_bytes, void *stream);

@@ -248,17 +248,18 @@ int w4a8_workspace(int M, int Kp, size_t given_bytes, hipStream_t s, char **ws) 
   return take_workspace(w4a8_ws_bytes(M, Kp), given_bytes, s, ws);
 }
 
-// bf16x3 GEMM on t16 (or, f8, t16f8) weights: split the activations into `ws`,
-// then the GEMM.
-int run_bf3(int fmt, const lbk::GemmArgs &a0, char *ws, hipStream_t s, bool f8 = false) {
-  int cus = 0;
+int current_cus() {
   DevInfo di;
-  if (device_info(&di) == 0) cus = di.cus;
+  return device_info(&di) == 0 ? di.cus : 0;
+}
+
+// bf16x3 GEMM on t16 (or, f8, t16f8) weights: split the activations into `ws`,
+// then the GEMM (with `prompt`, the prompt GEMM of that tile).
+int run_bf3(int fmt, const lbk::GemmArgs &a0, char *ws, const lbk::PromptTile *prompt, int cus, hipStream_t s,
+            bool f8 = false) {
   lbk::GemmArgs a = a0;
   a.x3 = reinterpret_cast<const uint4 *>(ws);
   hipError_t e;
-  lbk::PromptTile tile;
-  const bool prompt = lbk::prompt_tile_for(fmt, a.M, a.N, a.Kp, cus, &tile);
   if (fmt == lbk::F_W4A16) {
     // two float16 terms per row and its exponent (within the bf16x3 workspace)
     int *xexp = reinterpret_cast<int *>(ws + lbk::x2h_exp_offset(a.M, a.Kp));
@@ -271,24 +272,37 @@ int run_bf3(int fmt, const lbk::GemmArgs &a0, char *ws, hipStream_t s, bool f8 =
   }
   if (e != hipSuccess) return fail_hip(e, "activation split launch");
   if (!prompt) e = lbk::launch_bf3_gemm(fmt, a, cus, s, f8);
-  else if (fmt == lbk::F_W4A16) e = lbk::launch_w4a16_prompt(a, tile, f8, s);
-  else e = lbk::launch_mxfp4_prompt(a, tile, s);
+  else if (fmt == lbk::F_W4A16) e = lbk::launch_w4a16_prompt(a, *prompt, f8, s);
+  else e = lbk::launch_mxfp4_prompt(a, *prompt, s);
   if (e != hipSuccess) return fail_hip(e, "bf16x3 GEMM launch");
   return ok(LB_ISA_GFX950_MFMA);
 }
 
 // The workspace of a bf16x3 call: the split activations, then (K split over the
-// workgroups, where the shape takes it) the slices' partial outputs. A caller's
-// workspace of at least lbd_bf16x3_workspace_bytes bytes runs the unsplit GEMM; one
-// of lbd_bf16x3_workspace_bytes_split bytes, or none (the per-thread buffer), the
-// split one. The two give results within the same bound, not the same bits.
+// workgroups, where the shape takes it) the slices' partial outputs, or the digits of
+// MXFP4's prompt GEMM. A caller's workspace of at least lbd_bf16x3_workspace_bytes bytes
+// runs the unsplit GEMM (MXFP4: the batch kernel); one of
+// lbd_bf16x3_workspace_bytes_split bytes, or none (the per-thread buffer), the split one
+// or the prompt GEMM. They give results within the same bound, not the same bits.
+size_t bf3_room(int fmt, int M, int N, int Kp, int cus) {
+  const size_t room = align256(lbk::x3_bytes(M, Kp)) + lbk::bf3_part_bytes(fmt, M, N, Kp);
+  lbk::PromptTile tile;
+  return fmt == lbk::F_MXFP4 && lbk::prompt_tile_for(fmt, M, N, Kp, cus, &tile)
+             ? std::max(room, align256(lbk::digit_bytes(M, Kp)))
+             : room;
+}
+
 int bf3_call(int fmt, lbk::GemmArgs &a, char *ws, size_t given, hipStream_t s, bool f8 = false) {
+  const int cus = current_cus();
   const size_t x3 = align256(lbk::x3_bytes(a.M, a.Kp)), part = lbk::bf3_part_bytes(fmt, a.M, a.N, a.Kp);
   const bool own = ws == nullptr;
-  const int rc = take_workspace(own ? x3 + part : lbk::x3_bytes(a.M, a.Kp), given, s, &ws);
+  const int rc = take_workspace(own ? bf3_room(fmt, a.M, a.N, a.Kp, cus) : lbk::x3_bytes(a.M, a.Kp), given, s, &ws);
   if (rc < 0) return rc;
   if (part && (own || given >= x3 + part)) a.ypart = reinterpret_cast<float *>(ws + x3);
-  return run_bf3(fmt, a, ws, s, f8);
+  lbk::PromptTile tile;
+  const bool prompt = lbk::prompt_tile_for(fmt, a.M, a.N, a.Kp, cus, &tile) &&
+                      (fmt != lbk::F_MXFP4 || own || given >= lbk::digit_bytes(a.M, a.Kp));
+  return run_bf3(fmt, a, ws, prompt ? &tile : nullptr, cus, s, f8);
 }
 
 // Shared checks of the t16 GEMM entry points (32-bit offsets inside the kernels).
@@ -569,7 +583,7 @@ size_t lbd_bf16x3_workspace_bytes(int M, int Kp) {
 
 size_t lbd_bf16x3_workspace_bytes_split(int kind, int M, int N, int Kp) {
   if (M <= 0 || N <= 0 || Kp <= 0 || (kind != 0 && kind != 1)) return 0;
-  return align256(lbk::x3_bytes(M, Kp)) + lbk::bf3_part_bytes(kind == 1 ? lbk::F_MXFP4 : lbk::F_W4A16, M, N, Kp);
+  return bf3_room(kind == 1 ? lbk::F_MXFP4 : lbk::F_W4A16, M, N, Kp, current_cus());
 }
 
 int lbd_gemm_w4a16_t16(const float *x, int M, int Kp, const uint8_t *qwt, const float *st, const uint8_t *zt,

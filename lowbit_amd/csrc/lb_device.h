@@ -231,6 +231,18 @@ __device__ __forceinline__ void split3(float x, uint32_t &hi, uint32_t &mid, uin
   lo = bf16_rne(r1 - __uint_as_float(mid));
 }
 
+// The same of two elements with the conversion instruction, each term of both as bf16x2.
+__device__ __forceinline__ void split3_pair(float a, float b, uint32_t &hi, uint32_t &mid, uint32_t &lo) {
+  const auto cvt = [](float x, float y) {
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(v2f{x, y}, v2bf));
+  };
+  const auto rest = [](float x, uint32_t t) { return x - __uint_as_float(t); };
+  hi = cvt(a, b);
+  a = rest(a, hi << 16), b = rest(b, hi & 0xFFFF0000u);
+  mid = cvt(a, b);
+  lo = cvt(rest(a, mid << 16), rest(b, mid & 0xFFFF0000u));
+}
+
 // Two float32 values whose low 16 bits are zero (or may be dropped exactly) ->
 // bf16x2 with `a` in the low half.
 __device__ __forceinline__ uint32_t pack_bf16(uint32_t a, uint32_t b) {

@@ -154,8 +154,9 @@ bool prompt_tile_for(int fmt, int M, int N, int Kp, int num_cus, PromptTile *out
 // activations.
 hipError_t launch_w4a8_prompt(const GemmArgs &a, PromptTile t, hipStream_t s);
 // MXFP4 with many rows (lb_prompt.hip): the activations as kDigits E2M3 digits per
-// element (digit_bytes(M, Kp) bytes, within x3_bytes), the GEMM on them and t16 weights.
-constexpr int kDigits = 7;
+// element and their scales (digit_bytes(M, Kp) bytes), the GEMM on them, the activations
+// themselves (blocks that the digits do not hold) and t16 weights.
+constexpr int kDigits = 8;
 size_t digit_bytes(int M, int Kp);
 hipError_t launch_split_digits(const float *x, int M, int Kp, void *out, hipStream_t s);
 hipError_t launch_mxfp4_prompt(const GemmArgs &a, PromptTile t, hipStream_t s);

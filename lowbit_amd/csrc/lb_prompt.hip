@@ -249,106 +249,105 @@ hipError_t launch_w4a8_prompt(const GemmArgs &a, PromptTile t, hipStream_t s) {
 // their E8M0 block scales as they are, a 128-element group per instruction, at four
 // times the bf16 rate when the other operand is 6 bits wide. So the weights need no
 // decode at all, and each activation becomes kDigits signed digits of E2M3, which holds
-// every integer of [-16, 16] (times 1/8): with 2^ex above the largest |x| of its block
-// of 32, x 2^(4 - ex) = d1 + d2 2^-5 + d3 2^-10 ..., d1 = rint of it, and so on with the
-// exact remainders, the powers of two in the activations' own E8M0 scales. Seven digits
-// hold every element within 2^10 of its block's largest exactly and the others to
-// 2^-35 of 2^ex; a block where four or more elements lose bits to that (an outlier among
-// ordinary elements; normal ones hardly ever do, 2e-7 of blocks) is marked, and the GEMM makes
-// the further digits it takes from the activations themselves. Products and their sums over a group are exact up to the float32
-// accumulator. The leading digits add to one accumulator and the other six, 2^-5 of its
-// size, to a second, so that Y sees one float32 rounding per group.
+// every integer of [-16, 16] and every even one of [-32, 32] (times 1/8): with 2^ex above
+// the largest |x| of its block of 32, x 2^(5 - ex) = d1 + d2 2^-5 + d3 2^-10 ..., d1 the
+// nearest such integer, and so on with the exact remainders (at most 1/2 where |d| <= 16
+// and 1 elsewhere, so that the next digit is within 32 again), the powers of two in the
+// activations' own E8M0 scales. Eight digits reach 2^(ex - 40), which is the last bit of
+// any float32 from 2^(ex - 17) on: a block with no nonzero element below that is held
+// exactly. (A remainder above 1/2 goes back to a first
+// digit above 16, whose element ends 24 bits below its leading one, within five digits.)
+//
+// Other blocks (an element further below its block's largest: 9e-4 of the blocks of normal
+// activations with a few channels 8 times the rest; 1e-2 where those are 512 times the
+// rest; blocks whose digits' scales would run out; infinities and NaN) are marked, their
+// digits are zeros, and the GEMM takes them from the activations as the batch kernel does,
+// in three bf16 terms. What a block becomes depends on its own elements only. Products and
+// their sums over a group are exact up to the float32 accumulator. The leading digits add
+// to one accumulator and the other seven, 2^-5 of its size, to a second, so that Y sees one
+// float32 rounding per group.
+//
+// (Seven digits with marks only where four elements lost bits dropped small elements beside
+// a large one. Marks on every loss take 80 % of the 16-row groups of normal activations with
+// seven digits, 5 % with eight.)
 //
 // Digit tile of (row block, group, digit): lane 16 q + c holds row c, block 4 g + q, slots
 // 2 j / 2 j + 1 = elements j / j + 16 (the nibbles of byte j of the packed weights),
-// 24 bytes as 16 (1 KiB for the wave) then 8 (512 B); then 8 bytes per lane, the digits'
-// E8M0 scales and the mark.
-constexpr int kDigitTile = kWave * 24, kDigitBlock = kDigits * kDigitTile + kWave * 8;
-static_assert(kDigitBlock == 11 * 1024, "the GEMM stages whole KiB");
-size_t digit_bytes(int M, int Kp) { return (size_t)((M + 15) / 16) * ((Kp + 127) / 128) * kDigitBlock; }
+// 24 bytes as 16 (1 KiB for the wave) then 8 (512 B), row blocks within a group. After all
+// digit tiles, a dword per lane of each (row block, group): the first digit's E8M0 scale;
+// after these, 8 bytes of each, groups within a row block: bit l the mark of lane l.
+constexpr int kDigitTile = kWave * 24, kDigitBlock = kDigits * kDigitTile, kDigitScale = kWave * 4;
+static_assert(kDigitBlock == 12 * 1024, "the GEMM stages whole KiB");
+__host__ __device__ inline size_t digit_blocks(int M, int Kp) {
+  return (size_t)((M + 15) / 16) * ((Kp + 127) / 128);
+}
+size_t digit_bytes(int M, int Kp) { return digit_blocks(M, Kp) * (kDigitBlock + kDigitScale + 8); }
 
 typedef float v16f __attribute__((ext_vector_type(16)));
+typedef float v32f __attribute__((ext_vector_type(32)));
 typedef unsigned int v6u __attribute__((ext_vector_type(6)));
 typedef int v8i __attribute__((ext_vector_type(8)));
 typedef unsigned int v2u __attribute__((ext_vector_type(2)));
 
-// A lane's block of 32 activations as digits: lo and hi hold its halves, times 2^(4 - ex),
-// less the digits taken so far, in units of the next one.
-struct DigitBlock {
-  v16f lo, hi;
-  int e8;    // biased exponent of the next digit's scale
-  bool bad;  // holds an infinity or NaN
-
-  __device__ __forceinline__ void load(const float *x, int M, int Kp, int row, int b) {
-    const Rsrc rx = make_rsrc(x, (uint32_t)((size_t)M * Kp * 4));
-    const uint32_t off = row < M && 32 * b < Kp ? (uint32_t)(((size_t)row * Kp + 32 * b) * 4) : 0xFFFFFF00u;
-    uint32_t top = 0;
-#pragma unroll
-    for (int i = 0; i < 8; i++) {
-      const float4 t = ld_f4(rx, off + 16 * i);
-      const float e[4] = {t.x, t.y, t.z, t.w};
-#pragma unroll
-      for (int k = 0; k < 4; k++) {
-        top = max(top, __float_as_uint(e[k]) & 0x7FFFFFFFu);
-        if (i < 4) lo[4 * i + k] = e[k];
-        else hi[4 * (i - 4) + k] = e[k];
-      }
-    }
-    int ex = 0;
-    (void)frexpf(__uint_as_float(top), &ex);  // top < 2^ex
-    bad = top >= 0x7F800000u;
-#pragma unroll
-    for (int i = 0; i < 16; i++) lo[i] = ldexpf(lo[i], 4 - ex), hi[i] = ldexpf(hi[i], 4 - ex);
-    e8 = 127 + ex - 4 + 3;  // the first digit counts units of 2^(ex - 4), the tiles hold eighths
-  }
-  // the next digits, six bits each; zeros below the smallest scale
-  __device__ __forceinline__ v6u next() {
-    v16f dl, dh;
-#pragma unroll
-    for (int i = 0; i < 16; i++) {
-      dl[i] = __builtin_rintf(lo[i]);
-      dh[i] = __builtin_rintf(hi[i]);
-      lo[i] = (lo[i] - dl[i]) * 32.0f;
-      hi[i] = (hi[i] - dh[i]) * 32.0f;
-      if (e8 < 0) dl[i] = 0.0f, dh[i] = 0.0f;
-    }
-    e8 -= 5;
-    return __builtin_amdgcn_cvt_scalef32_2xpk16_fp6_f32(dl, dh, 8.0f);
-  }
-  // elements that the digits so far do not hold exactly
-  __device__ __forceinline__ int inexact() const {
-    int n = 0;
-#pragma unroll
-    for (int i = 0; i < 16; i++) n += (lo[i] != 0.0f) + (hi[i] != 0.0f);
-    return n;
-  }
-};
-
-// One wave per (row block, group), one lane per (row, block). An infinity or NaN makes
-// its block's scales NaN (255), so the row's outputs are NaN, as in the bf16 split.
+// One wave per (row block, group), one lane per (row, block).
 __global__ __launch_bounds__(kPThreads) void split_digits_kernel(const float *__restrict__ x, int M, int Kp,
                                                                  char *__restrict__ out) {
   const int lane = threadIdx.x & (kWave - 1), G = (Kp + 127) / 128, mblocks = (M + 15) / 16;
-  const size_t item = (size_t)blockIdx.x * kPWaves + threadIdx.x / kWave;
-  if (item >= (size_t)mblocks * G) return;  // whole waves only
+  const size_t items = (size_t)mblocks * G, item = (size_t)blockIdx.x * kPWaves + threadIdx.x / kWave;
+  if (item >= items) return;  // whole waves only
   const int mb = (int)(item % mblocks), g = (int)(item / mblocks);
-  DigitBlock d;
-  d.load(x, M, Kp, 16 * mb + (lane & 15), 4 * g + (lane >> 4));
-  char *dst = out + item * kDigitBlock;
-  uint32_t sc[2] = {0, 0};
+  const int row = 16 * mb + (lane & 15), b = 4 * g + (lane >> 4);
+  const Rsrc rx = make_rsrc(x, (uint32_t)((size_t)M * Kp * 4));
+  const uint32_t off = row < M && 32 * b < Kp ? (uint32_t)(((size_t)row * Kp + 32 * b) * 4) : 0xFFFFFF00u;
+  v16f lo, hi;  // the block's halves, then their remainders in units of the next digit
+  uint32_t top = 0, low = 0x7F800000u;  // largest magnitude, smallest nonzero one
 #pragma unroll
+  for (int i = 0; i < 8; i++) {
+    const float4 t = ld_f4(rx, off + 16 * i);
+    const float e[4] = {t.x, t.y, t.z, t.w};
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      const uint32_t u = __float_as_uint(e[k]) & 0x7FFFFFFFu;
+      top = max(top, u);
+      low = min(low, u ? u : 0x7F800000u);
+      if (i < 4) lo[4 * i + k] = e[k];
+      else hi[4 * (i - 4) + k] = e[k];
+    }
+  }
+  int ex = 0;
+  (void)frexpf(__uint_as_float(top), &ex);  // top < 2^ex
+  // the eighth digit's scale, 2^(ex - 37) in E8M0, must be one
+  const bool mark = top >= 0x7F800000u || (top && (ex < -90 || low < __float_as_uint(ldexpf(1.0f, ex - 17))));
+  if (mark || !top) ex = 0;
+#pragma unroll
+  for (int i = 0; i < 16; i++) {
+    lo[i] = mark ? 0.0f : ldexpf(lo[i], 5 - ex);
+    hi[i] = mark ? 0.0f : ldexpf(hi[i], 5 - ex);
+  }
+  char *dst = out + item * kDigitBlock;
+  // (a loop: unrolled, fetching its code takes most of a small call's time)
+#pragma unroll 1
   for (int t = 0; t < kDigits; t++) {
-    sc[t / 4] |= (d.bad ? 255u : (uint32_t)max(d.e8, 0)) << (8 * (t % 4));
-    const v6u p = d.next();
+    const v6u p = __builtin_amdgcn_cvt_scalef32_2xpk16_fp6_f32(lo, hi, 8.0f);
+    const v32f d = __builtin_amdgcn_cvt_scalef32_pk32_f32_fp6(p, 8.0f);
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+      lo[i] = (lo[i] - d[2 * i]) * 32.0f;
+      hi[i] = (hi[i] - d[2 * i + 1]) * 32.0f;
+    }
     *reinterpret_cast<uint4 *>(dst + t * kDigitTile + lane * 16) = make_uint4(p[0], p[1], p[2], p[3]);
     *reinterpret_cast<uint2 *>(dst + t * kDigitTile + 1024 + lane * 8) = make_uint2(p[4], p[5]);
   }
-  if (!d.bad && d.inexact() >= 4) sc[1] |= 1u << 24;
-  *reinterpret_cast<uint2 *>(dst + kDigits * kDigitTile + lane * 8) = make_uint2(sc[0], sc[1]);
+  // digit t + 1 counts units of 2^(ex - 5 - 5 t), the tiles hold eighths: scale 2^(ex - 2 - 5 t)
+  char *scales = out + items * kDigitBlock;
+  *reinterpret_cast<uint32_t *>(scales + item * kDigitScale + lane * 4) = (uint32_t)(127 + ex - 2);
+  const unsigned long long marks = __ballot(mark);
+  if (lane == 0)
+    reinterpret_cast<unsigned long long *>(scales + items * kDigitScale)[(size_t)mb * G + g] = marks;
 }
 
 hipError_t launch_split_digits(const float *x, int M, int Kp, void *out, hipStream_t s) {
-  const size_t items = (size_t)((M + 15) / 16) * ((Kp + 127) / 128);
+  const size_t items = digit_blocks(M, Kp);
   hipLaunchKernelGGL(split_digits_kernel, dim3((unsigned)((items + kPWaves - 1) / kPWaves)), dim3(kPThreads), 0, s, x,
                      M, Kp, static_cast<char *>(out));
   return hipGetLastError();
@@ -367,9 +366,9 @@ __device__ __forceinline__ v4f mx_product(int sel, v8i x, int sx, uint4 w4, int 
 
 template <int TM, int WN>
 __global__ __launch_bounds__(kPThreads, 2) void mxfp4_prompt_kernel(GemmArgs a, int mt, int nt) {
-  constexpr int SK = TM * kDigitBlock / 1024;  // KiB of a stage
-  constexpr int PW = (SK + kPWaves - 1) / kPWaves;
+  constexpr int SK = TM * kDigitBlock / 1024, PW = SK / kPWaves;  // KiB of a stage, and of a wave's share
   __shared__ __align__(16) char xs0[SK * 1024], xs1[SK * 1024], xs2[SK * 1024];
+  __shared__ __align__(16) char es0[TM * kDigitScale], es1[TM * kDigitScale], es2[TM * kDigitScale];
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int q = lane >> 4, c = lane & 15;
@@ -378,7 +377,10 @@ __global__ __launch_bounds__(kPThreads, 2) void mxfp4_prompt_kernel(GemmArgs a, 
   if (!prompt_tile(mt, nt, tm, tn)) return;
   const int mb0 = tm * TM, s0 = (tn * kPWaves + wave) * WN;
   const uint32_t mblocks = (uint32_t)((M + 15) / 16);
-  const Rsrc rx = make_rsrc(a.x3, (uint32_t)min((size_t)mblocks * G * kDigitBlock, (size_t)0xFFFFFFF0u));
+  const uint32_t xbytes = mblocks * (uint32_t)G * (uint32_t)kDigitBlock;
+  const Rsrc rd = make_rsrc(a.x3, xbytes);
+  const Rsrc rse = make_rsrc(reinterpret_cast<const char *>(a.x3) + xbytes, mblocks * (uint32_t)G * (uint32_t)kDigitScale);
+  const Rsrc rx = make_rsrc(a.x, (uint32_t)((size_t)M * Kp * 4));
   const Rsrc rw = make_rsrc(a.qw, (uint32_t)min(t16_qw_bytes(N, Kp), (size_t)0xFFFFFFF0u));
   const Rsrc re = make_rsrc(a.e8m0, (uint32_t)t16_e8m0_bytes(N, Kp));
 
@@ -388,18 +390,22 @@ __global__ __launch_bounds__(kPThreads, 2) void mxfp4_prompt_kernel(GemmArgs a, 
   } w0, w1, w2;
   // load `op` of this wave for group g: the first PW copy its share of the stage (row blocks
   // are consecutive within a group, so a stage is one run of KiB; past the last row block
-  // it reads the next group's, rows that are not stored, or zeros at the end), the others
-  // load its subtiles' weights and scales (past the last subtile: its columns are not stored)
-  constexpr int OPS = PW + 2 * WN;
-  const auto load = [&](int op, char *xd, Weights &n, int g) {
+  // it reads the next group's, rows that are not stored, or zeros at the end), the next a
+  // row block's scales (every wave one, so that all wait for as many loads), the others
+  // its subtiles' weights and scales (past the last subtile: its columns are not stored)
+  constexpr int OPS = PW + 1 + 2 * WN;
+  const auto load = [&](int op, char *xd, char *ed, Weights &n, int g) {
+    const uint32_t block = (uint32_t)g * mblocks + (uint32_t)mb0;
     if (op < PW) {
-      const int t = min(wave * PW + op, SK - 1);
-      lds_load16(rx, xd + t * 1024, (uint32_t)lane * 16u + ((uint32_t)g * mblocks + (uint32_t)mb0) * (uint32_t)kDigitBlock +
-                     (uint32_t)t * 1024u, 0);
+      const int t = wave * PW + op;
+      lds_load16(rd, xd + t * 1024, block * (uint32_t)kDigitBlock + (uint32_t)t * 1024u + (uint32_t)lane * 16u, 0);
+    } else if (op == PW) {
+      const int t = wave % TM;
+      lds_load4(rse, ed + t * kDigitScale, (block + t) * (uint32_t)kDigitScale + (uint32_t)lane * 4u, 0);
     } else if (op < OPS) {
-      const int j = (op - PW) >> 1;
+      const int j = (op - PW - 1) >> 1;
       const uint32_t sj = (uint32_t)min(s0 + j, S - 1);
-      if ((op - PW) & 1) n.e[j] = __builtin_amdgcn_raw_buffer_load_b8(re, lane, (int)((sj * G4 + g) * 64u), 0);
+      if ((op - PW - 1) & 1) n.e[j] = __builtin_amdgcn_raw_buffer_load_b8(re, lane, (int)((sj * G4 + g) * 64u), 0);
       else n.w[j] = ld_b128(rw, (uint32_t)lane * 16u, (sj * G4 + g) * 1024u);
     }
   };
@@ -413,18 +419,23 @@ __global__ __launch_bounds__(kPThreads, 2) void mxfp4_prompt_kernel(GemmArgs a, 
   // occupies the matrix core for 16 cycles and the wave's issue for 8, so
   // what is issued one by one between products costs nothing, and in clumps its whole time;
   // every slot is pinned, as the scheduler would make clumps (and sink the loads to the end).
-  const auto group = [&](const char *xd, const Weights &n, char *nxd, Weights &nn, int g) {
+  const auto group = [&](const char *xd, const char *ed, const Weights &n, char *nxd, char *ned, Weights &nn, int g) {
     constexpr int K = TM * kDigits;  // step k: row block k / kDigits, digit k % kDigits
     v4i xa[3];
-    v2u xb[3], sc[2];
+    v2u xb[3];
+    uint32_t sc[2][2];
     const auto read_a = [&](int k) {
       xa[k % 3] = *reinterpret_cast<const v4i *>(xd + (k / kDigits) * kDigitBlock + (k % kDigits) * kDigitTile + lane * 16);
     };
     const auto read_b = [&](int k) {
       const char *blk = xd + (k / kDigits) * kDigitBlock;
       xb[k % 3] = *reinterpret_cast<const v2u *>(blk + (k % kDigits) * kDigitTile + 1024 + lane * 8);
-      if (k % kDigits == 0)
-        sc[(k / kDigits) & 1] = *reinterpret_cast<const v2u *>(blk + kDigits * kDigitTile + lane * 8);
+      if (k % kDigits == 0) {  // scales five apart, no borrow between bytes: the first is at least 35
+        uint32_t *p = sc[(k / kDigits) & 1];
+        const uint32_t e = *reinterpret_cast<const uint32_t *>(ed + (k / kDigits) * kDigitScale + lane * 4);
+        p[0] = __builtin_amdgcn_perm(e, e, 0u) - 0x0F0A0500u;
+        p[1] = p[0] - 0x14141414u;
+      }
     };
     read_a(0);
     read_b(0);
@@ -442,44 +453,152 @@ __global__ __launch_bounds__(kPThreads, 2) void mxfp4_prompt_kernel(GemmArgs a, 
         __builtin_amdgcn_sched_barrier(0);
         if (j == 0 && k + 2 < K) read_a(k + 2);
         if (j == 1 && k + 2 < K) read_b(k + 2);
-        if (j >= 2) load(op++, nxd, nn, min(g + 2, G - 1));
+        if (j >= 2) load(op++, nxd, ned, nn, min(g + 2, G - 1));
         __builtin_amdgcn_sched_barrier(0);
       }
     }
     static_assert(K * (WN - 2) >= OPS, "every load has a slot");
-#pragma unroll
-    for (int i = 0; i < TM; i++) {
-      if (!__any((int)(sc[i & 1][1] >> 24))) continue;
-      DigitBlock d;
-      d.load(a.x, M, Kp, 16 * (mb0 + i) + c, 4 * g + q);
-#pragma unroll 1
-      for (int t = 0; t < kDigits; t++) (void)d.next();
-      while (__any(!d.bad && d.e8 >= 0 && d.inexact() > 0)) {
-        const int sx = d.bad ? 255 : max(d.e8, 0);
-        const v6u p = d.next();
-        const v8i x = {(int)p[0], (int)p[1], (int)p[2], (int)p[3], (int)p[4], (int)p[5], 0, 0};
-#pragma unroll
-        for (int j = 0; j < WN; j++) lo[i][j] = mx_product(0, x, sx, n.w[j], (int)n.e[j], lo[i][j]);
-      }
-    }
   };
+  // the marks of groups g0 + lane (those of the first 64 groups are loaded ahead)
+  unsigned long long mine[TM];
+  const auto load_marks = [&](int g0) {
+    const auto *marks = reinterpret_cast<const unsigned long long *>(reinterpret_cast<const char *>(a.x3) + xbytes +
+                                                                     (size_t)mblocks * G * kDigitScale);
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+      mine[i] = mb0 + i < (int)mblocks && g0 + lane < G ? marks[(size_t)(mb0 + i) * G + g0 + lane] : 0;
+  };
+  load_marks(0);
+  __builtin_amdgcn_sched_barrier(0);
   // two groups are in flight ahead of the one that runs
 #pragma unroll
-  for (int op = 0; op < OPS; op++) load(op, xs0, w0, 0);
+  for (int op = 0; op < OPS; op++) load(op, xs0, es0, w0, 0);
   __builtin_amdgcn_sched_barrier(0);  // stage_ready counts on all of group 0's loads coming first
 #pragma unroll
-  for (int op = 0; op < OPS; op++) load(op, xs1, w1, min(1, G - 1));
+  for (int op = 0; op < OPS; op++) load(op, xs1, es1, w1, min(1, G - 1));
   __builtin_amdgcn_sched_barrier(0);
-  const auto step = [&](const char *xd, const Weights &n, char *nxd, Weights &nn, int g) {
+  const auto step = [&](const char *xd, const char *ed, const Weights &n, char *nxd, char *ned, Weights &nn, int g) {
     stage_ready<OPS>();
-    group(xd, n, nxd, nn, g);
+    group(xd, ed, n, nxd, ned, nn, g);
   };
   for (int g = 0; g < G; g += 3) {
-    step(xs0, w0, xs2, w2, g);
-    if (g + 1 < G) step(xs1, w1, xs0, w0, g + 1);
-    if (g + 2 < G) step(xs2, w2, xs1, w1, g + 2);
+    step(xs0, es0, w0, xs2, es2, w2, g);
+    if (g + 1 < G) step(xs1, es1, w1, xs0, es0, w0, g + 1);
+    if (g + 2 < G) step(xs2, es2, w2, xs1, es1, w1, g + 2);
   }
   stage_ready<0>();  // no load to LDS outlives the workgroup
+  // Marked blocks: weights, terms and order of the batch kernel (bf3_gemm_kernel), the terms
+  // of the other blocks zero, so that no row changes with the others of its row block. Apart
+  // from the loop above, whose registers they would spill. Up to 3 TM (row block, group)s at
+  // once: wave u makes their operands u in the stages' LDS, then every wave takes them all.
+  // (Little code: for a call of one round, fetching it is most of the cost.)
+  constexpr int R = 3 * TM;
+  const auto room = [&](int t) { return (t < TM ? xs0 : t < 2 * TM ? xs1 : xs2) + t % TM * kDigitBlock; };
+  for (int g0 = 0; g0 < G; g0 += kWave) {
+    if (g0 > 0) load_marks(g0);
+    unsigned long long todo[TM];
+#pragma unroll
+    for (int i = 0; i < TM; i++) todo[i] = __ballot(mine[i] != 0);
+    // the next of a list: row block i, group g0 + gl; false (and gl = 0) past its end
+    const auto next = [](unsigned long long (&t)[TM], int &i, int &gl) {
+      i = TM > 1 && !t[0];
+      const unsigned long long v = t[0] ? t[0] : t[TM - 1];
+      gl = v ? __builtin_ctzll(v) : 0;
+      if (TM > 1 && i) t[TM - 1] = v & (v - 1);
+      else t[0] = v & (v - 1);
+      return v != 0;
+    };
+    while (todo[0] | todo[TM - 1]) {
+      float4 l4[R], h4[R];
+      unsigned long long list[TM];
+      int count = 0, i, gl;
+#pragma unroll
+      for (int k = 0; k < TM; k++) list[k] = todo[k];
+#pragma unroll
+      for (int t = 0; t < R; t++) {
+        const bool some = next(list, i, gl);
+        count += some;
+        const unsigned long long m = i ? mine[TM - 1] : mine[0];
+        const uint32_t half = lane < 32 ? __builtin_amdgcn_readlane((uint32_t)m, gl)
+                                        : __builtin_amdgcn_readlane((uint32_t)(m >> 32), gl);
+        const bool mark = some && (half >> (lane & 31) & 1u);
+        // (a marked block is inside the activations)
+        const uint32_t off = (uint32_t)(((size_t)(16 * (mb0 + i) + c) * Kp + 128 * (g0 + gl) + 32 * q + 4 * wave) * 4);
+        l4[t] = ld_f4(rx, mark ? off : 0xFFFFFF00u);
+        h4[t] = ld_f4(rx, mark ? off + 64 : 0xFFFFFF00u);
+      }
+      const auto weights = [&](Weights &n, int g) {
+#pragma unroll
+        for (int op = PW + 1; op < OPS; op++) load(op, nullptr, nullptr, n, g);
+      };
+      Weights n;
+      next(todo, i, gl);
+      weights(n, g0 + gl);
+      __builtin_amdgcn_sched_barrier(0);
+      __syncthreads();
+#pragma unroll
+      for (int t = 0; t < R; t++) {
+        if (t >= count) break;
+        const float v[8] = {l4[t].x, h4[t].x, l4[t].y, h4[t].y, l4[t].z, h4[t].z, l4[t].w, h4[t].w};
+        uint32_t x3[3][4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) split3_pair(v[2 * k], v[2 * k + 1], x3[0][k], x3[1][k], x3[2][k]);
+#pragma unroll
+        for (int p = 0; p < 3; p++)
+          *reinterpret_cast<uint4 *>(room(t) + (wave * 3 + p) * 1024 + lane * 16) =
+              make_uint4(x3[p][0], x3[p][1], x3[p][2], x3[p][3]);
+      }
+      __syncthreads();
+#pragma unroll 1
+      for (int t = 0; t < count; t++) {
+        const Weights w = n;
+        const int it = i;
+        if (t + 1 < count) {
+          next(todo, i, gl);
+          weights(n, g0 + gl);
+        }
+        const char *xb = room(t) + lane * 16;
+        v4f d[WN];
+        float bs[WN], fs[WN];
+#pragma unroll
+        for (int j = 0; j < WN; j++) {
+          const int e = (int)w.e[j];
+          int emax = max(e, __shfl_xor(e, 16));
+          emax = max(emax, __shfl_xor(emax, 32));
+          bs[j] = e - emax >= -126 ? __uint_as_float((uint32_t)(e - emax + 127) << 23) : 0.0f;
+          fs[j] = e8m0_to_f32((uint32_t)emax);
+          d[j] = v4f{0.f, 0.f, 0.f, 0.f};
+        }
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+          v4u wb[WN];
+#pragma unroll
+          for (int j = 0; j < WN; j++) {
+            const uint32_t wu = u == 0 ? w.w[j].x : u == 1 ? w.w[j].y : u == 2 ? w.w[j].z : w.w[j].w;
+            wb[j] = v4u{__builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(wu, bs[j], 0)),
+                        __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(wu, bs[j], 1)),
+                        __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(wu, bs[j], 2)),
+                        __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(wu, bs[j], 3))};
+          }
+#pragma unroll
+          for (int p = 0; p < 3; p++) {
+            const v8bf x = *reinterpret_cast<const v8bf *>(xb + (u * 3 + p) * 1024);
+#pragma unroll
+            for (int j = 0; j < WN; j++)
+              d[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, __builtin_bit_cast(v8bf, wb[j]), d[j], 0, 0, 0);
+          }
+        }
+#pragma unroll
+        for (int k = 0; k < TM; k++) {
+          if (it != k) continue;
+#pragma unroll
+          for (int j = 0; j < WN; j++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) hi[k][j][r] = __builtin_fmaf(fs[j], d[j][r], hi[k][j][r]);
+        }
+      }
+    }
+  }
 #pragma unroll
   for (int i = 0; i < TM; i++) {
 #pragma unroll
@@ -673,10 +792,13 @@ hipError_t launch_w4a16_prompt(const GemmArgs &a, PromptTile t, bool f8, hipStre
 // a launch that leaves each CU one workgroup or less takes (a little more than) G times
 // its time per group however few rows there are, while the batch kernels' time falls with
 // the work; so the line is drawn in 16 x 16 tiles of Y per CU, T.
-//   MXFP4  0.72 us a group; 0.55 with 16-row tiles, taken while they fill one round of the
-//          CUs (256 x 4096 x 4096 29.5 -> 26.0). Wins from T = 12 at every K
-//          (192 x 4096 x 4096 38.8 -> 25.9, x 11008 87.8 -> 56.2, 1024 x 4096 x 4096 179 ->
-//          61; 128 rows 19.5 against 25.0, not taken).
+//   MXFP4  about 11 us + 0.68 a group with 16-row tiles, taken while they fill one round of
+//          the CUs, 12.5 + 0.97 a group and round with 32-row ones, against 8 us + 1.0-1.1 a
+//          group of the batch kernel up to T = 22, 1.5 at 24, 0.06 T above (normal activations
+//          with a few large channels): 192 x 4096 x 4096 40.7 -> 32.2, 448 x 4096 x 4096
+//          64.5 -> 46.1, 1024 x 4096 x 4096 179 -> 80, 33 x 28672 x 8192 93.3 -> 72.5, 1024
+//          x 4096 x 11008 448 -> 187. Not taken: 192 x 4096 x 1024 15.4 against 16.3, 112 x
+//          11008 x 4096 (T = 19) 40.3 against 44.3, 208 x 9728 x 896 (T = 31) 20.6 against 24.2.
 //   W4A16  1.13 us a group and round of 256 workgroups against 0.055 T of the batch kernel
 //          (512 x 4096 x 4096 60.5 -> 49.0, 2048 x 11008 x 4096 642 -> 364; 256 x 4096 x
 //          4096 39.9 against 44.4, not taken).
@@ -696,8 +818,9 @@ bool prompt_tile_for(int fmt, int M, int N, int Kp, int num_cus, PromptTile *out
   };
   PromptTile t;
   if (fmt == F_MXFP4) {
-    if (T < 12) return false;
     t = PromptTile{rounds(1, 4) <= 1 ? 1 : 2, 4};
+    const bool gains = t.tm == 1 ? T >= 12 && G >= 9 : T >= 33 || (T >= 24 && G >= 8) || (T >= 17 && G >= 64);
+    if (!gains) return false;
   } else if (fmt == F_W4A16) {
     t = PromptTile{2, 4};
     if (1.13 * std::ceil(rounds(2, 4)) > 0.055 * T) return false;

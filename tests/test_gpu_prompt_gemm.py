@@ -15,9 +15,9 @@ from problems import outlier_int4_problem
 
 pytestmark = pytest.mark.gpu
 
-# M, N, K: ragged M and N, 1, 2, 3, 7 and 8 groups; 13 or more 16 x 16 tiles of Y per CU,
+# M, N, K: ragged M and N, 1, 2, 3, 7 and 8 groups; 33 or more 16 x 16 tiles of Y per CU,
 # where every format takes these kernels
-SHAPES = [(1041, 3100, 128), (645, 5003, 256), (300, 9728, 384), (500, 4030, 896), (2090, 2601, 1024)]
+SHAPES = [(1041, 3100, 128), (645, 5003, 256), (300, 9728, 384), (560, 4030, 896), (2090, 2601, 1024)]
 
 
 def _int4(rng, n, k, asym, zmax=15):
@@ -61,7 +61,8 @@ def test_w4a16(rng, m, n, k, asym, zmax):
         np.testing.assert_array_equal(dy.to_array((m, n), np.float32), y)
 
 
-@pytest.mark.parametrize("m,n,k", SHAPES + [(200, 4100, 32), (777, 4096, 1056)])
+# MXFP4 also: a last group of one block; 16-row tiles with every number of groups left over
+@pytest.mark.parametrize("m,n,k", SHAPES + [(777, 4096, 1056), (200, 4100, 1152), (190, 4090, 1280), (235, 4089, 1408)])
 def test_mxfp4(rng, m, n, k):
     W = lb.MXFP4Weights(rng.integers(0, 256, (n, k // 2), dtype=np.uint8),
                         rng.integers(117, 131, (n, k // 32), dtype=np.uint8), k)
@@ -99,3 +100,93 @@ def test_columns_that_take_nothing_from_huge_elements(rng):
         x = rng.standard_normal((m, k)).astype(np.float32)
         x[::2, huge] *= np.float32(amp)
         O.assert_fp_close(K.gemm_mxfp4(x, D), O.gemm_mxfp4_ref(x, W.qw, W.e8m0), O.fp_bound(x, W.dequantize()), 1e-5)
+
+
+# one 32-row and one 16-row tile shape (see lb_prompt.hip, prompt_tile_for)
+MX_SHAPES = [(640, 4096, 512), (200, 4100, 1280)]
+
+
+def _mx_limit(x, W, y):
+    """Largest error over the bound, with no absolute floor."""
+    ref, bound = O.gemm_mxfp4_ref(x, W.qw, W.e8m0), O.fp_bound(x, W.dequantize())
+    return (np.abs(y.astype(np.float64) - ref) / (1e-5 * bound + 1e-300)).max()
+
+
+@pytest.mark.parametrize("m,n,k", MX_SHAPES)
+@pytest.mark.parametrize("small", [1, 2, 3, 31])
+@pytest.mark.parametrize("amp", [1e6, 1e9, 1e12, 3e38])
+def test_mxfp4_small_elements_beside_a_large_one(rng, m, n, k, small, amp):
+    """A large element that meets zero weights, `small` ordinary or tiny ones and zeros in
+    each block of 32: the products of the small ones must keep the bound."""
+    x = np.zeros((m, k // 32, 32), np.float32)
+    x[:, :, 0] = amp
+    x[:, :, 1:1 + small] = rng.standard_normal((m, k // 32, small))
+    x[::3, :, 1:1 + small] *= 1e-10
+    x = x.reshape(m, k)
+    codes = rng.integers(0, 16, (n, k), dtype=np.uint8)
+    codes[:, ::32] = 0
+    W = lb.MXFP4Weights(lb.formats.pack_nibbles(codes, 32), rng.integers(122, 128, (n, k // 32), dtype=np.uint8), k)
+    assert _mx_limit(x, W, K.gemm_mxfp4(x, lb.to_device(W))) <= 1.0
+
+
+@pytest.mark.parametrize("m,n,k", MX_SHAPES)
+@pytest.mark.parametrize("mag", [1e-36, 1e-33, 1e-30, 1e-10, 1e10, 1e30])
+def test_mxfp4_activation_magnitudes(rng, m, n, k, mag):
+    """test_gpu_random_shapes.test_activation_magnitudes at prompt sizes."""
+    W = lb.quantize_mxfp4(rng.standard_normal((n, k)).astype(np.float32))
+    x = (rng.standard_normal((m, k)) * mag).astype(np.float32)
+    assert _mx_limit(x, W, K.gemm_mxfp4(x, lb.to_device(W))) <= 1.0
+
+
+@pytest.mark.parametrize("m,n,k", MX_SHAPES)
+@pytest.mark.parametrize("mag", [1e-20, 1.0, 1e30])
+def test_mxfp4_keeps_every_bit_of_an_activation(rng, m, n, k, mag):
+    """Weight rows with a single 1: y[i, j] is the activation x[i, j % k] itself, normal or
+    log-uniform over 2^40, whatever its neighbours are. (All above 2^-110: below it the last
+    of an activation's three bf16 terms would be a subnormal, which the matrix cores flush,
+    2^-16 of the element at the most, in the batch kernel as here.)"""
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    x[m // 2:] *= np.exp2(rng.uniform(-20, 20, x[m // 2:].shape)).astype(np.float32)
+    x *= np.float32(mag)
+    codes = np.zeros((n, k), np.uint8)
+    codes[np.arange(n), np.arange(n) % k] = 2  # E2M1 1.0
+    W = lb.MXFP4Weights(lb.formats.pack_nibbles(codes, 32), np.full((n, k // 32), 127, np.uint8), k)
+    np.testing.assert_array_equal(K.gemm_mxfp4(x, lb.to_device(W)), x[:, np.arange(n) % k])
+
+
+@pytest.mark.parametrize("m,n,k", MX_SHAPES)
+def test_mxfp4_rows_do_not_depend_on_each_other(rng, m, n, k):
+    """Outliers, tiny values, infinities and NaN in some rows leave the others' bits alone
+    (weight rows with few nonzeros, so that the lowest bits of an activation show)."""
+    codes = rng.integers(0, 16, (n, k), dtype=np.uint8) * (rng.random((n, k)) < 2 / k).astype(np.uint8)
+    W = lb.MXFP4Weights(lb.formats.pack_nibbles(codes, 32), rng.integers(120, 130, (n, k // 32), dtype=np.uint8), k)
+    D = lb.to_device(W)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    x[m // 2:, ::5] *= np.exp2(rng.uniform(-30, 10, (m - m // 2, (k + 4) // 5))).astype(np.float32)
+    y = K.gemm_mxfp4(x, D)
+    x2, hit = x.copy(), np.arange(m) % 7 == 3
+    x2[hit, ::9] *= 1e9
+    x2[3], x2[10, 4], x2[17, 5] = 1e-38, np.inf, np.nan
+    y2 = K.gemm_mxfp4(x2, D)
+    np.testing.assert_array_equal(y2[~hit], y[~hit])
+    assert not np.array_equal(y2[hit], y[hit])
+
+
+def test_mxfp4_workspace_without_room_for_the_digits_takes_the_batch_kernel(rng):
+    """A workspace of lbd_bf16x3_workspace_bytes is accepted and meets the bound; one of
+    lbd_bf16x3_workspace_bytes_split gives the bits of the library's own."""
+    m, n, k = MX_SHAPES[0]
+    W = lb.quantize_mxfp4(rng.standard_normal((n, k)).astype(np.float32))
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    qt, et = lb.to_device(W).tiles()
+    L, prm = K.lib(), K._Params(-1, 0, 0, 0, 0, 0, 0)
+    dx = K.DeviceBuffer.from_array(x)
+    ys = []
+    for nb in (0, L.lbd_bf16x3_workspace_bytes_split(1, m, n, k), L.lbd_bf16x3_workspace_bytes(m, k)):
+        dy, ws = K.DeviceBuffer(m * n * 4), K.DeviceBuffer(nb + 256) if nb else None
+        assert L.lbd_gemm_mxfp4_t16(dx.ptr, m, k, qt.ptr, et.ptr, n, dy.ptr, C.byref(prm), ws.ptr if ws else None, nb,
+                                    None) == K.ISA_GFX950_MFMA
+        ys.append(dy.to_array((m, n), np.float32))
+        assert _mx_limit(x, W, ys[-1]) <= 1.0
+    np.testing.assert_array_equal(ys[0], ys[1])
+    assert not np.array_equal(ys[0], ys[2])
