@@ -273,9 +273,10 @@ int lbd_repack_mxfp4_t16(const uint8_t *qw, const uint8_t *e8m0, int N, int Kp,
 /* y = x . w^T as lbd_gemm_mxfp4 on t16 weights, the bf16 matrix-core path of
  * lbd_gemm_w4a16_t16 (block scales 2^(e - 127) exact; E8M0 255 gives NaN). With many
  * rows it runs on the MX matrix instruction instead, which takes the weights as they
- * are: blocks of 32 activations whose nonzero magnitudes lie within 2^17 of each other
- * become 8 six-bit digits per element, which hold them exactly; other blocks go through
- * the three bf16 terms. A workspace of lbd_bf16x3_workspace_bytes_split bytes, or NULL. */
+ * are: a block of 32 activations with no nonzero magnitude below 2^(ex - 17), 2^ex above
+ * its largest, becomes 8 six-bit digits per element, which hold it exactly; other blocks go
+ * through the three bf16 terms. That takes a workspace of
+ * lbd_bf16x3_workspace_bytes_split bytes, or NULL, and y apart from x. */
 int lbd_gemm_mxfp4_t16(const float *x, int M, int Kp, const uint8_t *qwt,
                        const uint8_t *et, int N, float *y, const lb_params *p,
                        void *workspace, size_t workspace_bytes, void *stream);

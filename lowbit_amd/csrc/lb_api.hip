@@ -299,9 +299,12 @@ int bf3_call(int fmt, lbk::GemmArgs &a, char *ws, size_t given, hipStream_t s, b
   const int rc = take_workspace(own ? bf3_room(fmt, a.M, a.N, a.Kp, cus) : lbk::x3_bytes(a.M, a.Kp), given, s, &ws);
   if (rc < 0) return rc;
   if (part && (own || given >= x3 + part)) a.ypart = reinterpret_cast<float *>(ws + x3);
+  // MXFP4's prompt GEMM reads the activations while other workgroups store Y; the other
+  // kernels only read their split, so there Y may lie on X
+  const bool apart = a.x + (size_t)a.M * a.Kp <= a.y || a.y + (size_t)a.M * a.N <= a.x;
   lbk::PromptTile tile;
   const bool prompt = lbk::prompt_tile_for(fmt, a.M, a.N, a.Kp, cus, &tile) &&
-                      (fmt != lbk::F_MXFP4 || own || given >= lbk::digit_bytes(a.M, a.Kp));
+                      (fmt != lbk::F_MXFP4 || (apart && (own || given >= lbk::digit_bytes(a.M, a.Kp))));
   return run_bf3(fmt, a, ws, prompt ? &tile : nullptr, cus, s, f8);
 }
 

@@ -172,6 +172,29 @@ def test_mxfp4_rows_do_not_depend_on_each_other(rng, m, n, k):
     assert not np.array_equal(y2[hit], y[hit])
 
 
+@pytest.mark.parametrize("shift", [0, 1])
+def test_mxfp4_y_on_x(rng, shift):
+    """Y may lie on X (N = K), or begin in X's last row: marked blocks are read from X while
+    Y is stored, so such a call takes the batch kernel, which is done with X by then."""
+    m, n = 1040, 2048
+    W = lb.quantize_mxfp4(rng.standard_normal((n, n)).astype(np.float32))
+    x = rng.standard_normal((m, n)).astype(np.float32)
+    x[:, ::9] *= 1e9
+    qt, et = lb.to_device(W).tiles()
+    L, prm = K.lib(), K._Params(-1, 0, 0, 0, 0, 0, 0)
+    def call(px, py, nb):
+        ws = K.DeviceBuffer(nb)
+        assert L.lbd_gemm_mxfp4_t16(px, m, n, qt.ptr, et.ptr, n, py, C.byref(prm), ws.ptr, nb,
+                                    None) == K.ISA_GFX950_MFMA
+    dx, dy = K.DeviceBuffer.from_array(x), K.DeviceBuffer(m * n * 4)
+    call(dx.ptr, dy.ptr, L.lbd_bf16x3_workspace_bytes(m, n))
+    both = K.DeviceBuffer.from_array(np.concatenate([x, np.zeros_like(x)]))
+    off = shift * (m - 1) * n
+    call(both.ptr, both.ptr + 4 * off, L.lbd_bf16x3_workspace_bytes_split(1, m, n, n))
+    got = both.to_array((2 * m * n,), np.float32)[off:off + m * n].reshape(m, n)
+    np.testing.assert_array_equal(got, dy.to_array((m, n), np.float32))
+
+
 def test_mxfp4_workspace_without_room_for_the_digits_takes_the_batch_kernel(rng):
     """A workspace of lbd_bf16x3_workspace_bytes is accepted and meets the bound; one of
     lbd_bf16x3_workspace_bytes_split gives the bits of the library's own."""
