@@ -405,7 +405,7 @@ __global__ __launch_bounds__(kPThreads, 2) void mxfp4_prompt_kernel(GemmArgs a, 
     } else if (op < OPS) {
       const int j = (op - PW - 1) >> 1;
       const uint32_t sj = (uint32_t)min(s0 + j, S - 1);
-      if ((op - PW - 1) & 1) n.e[j] = __builtin_amdgcn_raw_buffer_load_b8(re, lane, (int)((sj * G4 + g) * 64u), 0);
+      if ((op - PW - 1) & 1) n.e[j] = ld_u32(re, (uint32_t)(lane & ~3), (sj * G4 + g) * 64u);
       else n.w[j] = ld_b128(rw, (uint32_t)lane * 16u, (sj * G4 + g) * 1024u);
     }
   };
@@ -441,6 +441,9 @@ __global__ __launch_bounds__(kPThreads, 2) void mxfp4_prompt_kernel(GemmArgs a, 
     read_b(0);
     read_a(1);
     read_b(1);
+    int sw[WN];  // the lane's byte of its dword of scales (the instruction reads the lowest)
+#pragma unroll
+    for (int j = 0; j < WN; j++) sw[j] = (int)(n.e[j] >> (8 * (lane & 3)));
     int op = 0;
 #pragma unroll
     for (int k = 0; k < K; k++) {
@@ -449,7 +452,7 @@ __global__ __launch_bounds__(kPThreads, 2) void mxfp4_prompt_kernel(GemmArgs a, 
 #pragma unroll
       for (int j = 0; j < WN; j++) {
         v4f &o = t == 0 ? hi[i][j] : lo[i][j];
-        o = mx_product(t & 3, x, (int)sc[i & 1][t >> 2], n.w[j], (int)n.e[j], o);
+        o = mx_product(t & 3, x, (int)sc[i & 1][t >> 2], n.w[j], sw[j], o);
         __builtin_amdgcn_sched_barrier(0);
         if (j == 0 && k + 2 < K) read_a(k + 2);
         if (j == 1 && k + 2 < K) read_b(k + 2);
@@ -481,11 +484,16 @@ __global__ __launch_bounds__(kPThreads, 2) void mxfp4_prompt_kernel(GemmArgs a, 
     stage_ready<OPS>();
     group(xd, ed, n, nxd, ned, nn, g);
   };
-  for (int g = 0; g < G; g += 3) {
+  // (no way into a step but from the one before it: where two meet, the compiler waits for
+  // the loads that either has in flight)
+  int g = 0;
+  for (; g + 3 <= G; g += 3) {
     step(xs0, es0, w0, xs2, es2, w2, g);
-    if (g + 1 < G) step(xs1, es1, w1, xs0, es0, w0, g + 1);
-    if (g + 2 < G) step(xs2, es2, w2, xs1, es1, w1, g + 2);
+    step(xs1, es1, w1, xs0, es0, w0, g + 1);
+    step(xs2, es2, w2, xs1, es1, w1, g + 2);
   }
+  if (g < G) step(xs0, es0, w0, xs2, es2, w2, g);
+  if (g + 1 < G) step(xs1, es1, w1, xs0, es0, w0, g + 1);
   stage_ready<0>();  // no load to LDS outlives the workgroup
   // Marked blocks: weights, terms and order of the batch kernel (bf3_gemm_kernel), the terms
   // of the other blocks zero, so that no row changes with the others of its row block. Apart
@@ -562,7 +570,7 @@ __global__ __launch_bounds__(kPThreads, 2) void mxfp4_prompt_kernel(GemmArgs a, 
         float bs[WN], fs[WN];
 #pragma unroll
         for (int j = 0; j < WN; j++) {
-          const int e = (int)w.e[j];
+          const int e = (int)((w.e[j] >> (8 * (lane & 3))) & 0xFFu);
           int emax = max(e, __shfl_xor(e, 16));
           emax = max(emax, __shfl_xor(emax, 32));
           bs[j] = e - emax >= -126 ? __uint_as_float((uint32_t)(e - emax + 127) << 23) : 0.0f;

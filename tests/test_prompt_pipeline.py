@@ -57,3 +57,15 @@ def test_groups_loaded_ahead_are_apart(kernels):
         runs = [k for i, k in enumerate(kinds) if i == 0 or kinds[i - 1] != k]
         assert runs == ["lds", "weights", "lds", "weights"], (name, runs)
         assert kinds[:len(kinds) // 2] == kinds[len(kinds) // 2:], (name, kinds)
+
+
+def test_no_step_waits_for_the_loads_it_issued(kernels):
+    """In the loop, a step's loads are for two groups on; what it waits for before its own
+    first load must leave the previous step's in flight (some of them at least: it issues
+    8 or more after the ones that the step's first products need)."""
+    for name, code in kernels.items():
+        bars = [i for i, s in enumerate(code) if s.startswith("s_barrier")][:3]
+        for i in bars:  # the three steps of the loop
+            first = next(j for j in range(i, len(code)) if code[j].startswith("buffer_load"))
+            waits = [int(n) for s in code[i - 4:first] for n in re.findall(r"vmcnt\((\d+)\)", s)]
+            assert waits and min(waits) >= 8, (name, waits)
