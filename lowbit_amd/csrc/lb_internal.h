@@ -148,6 +148,21 @@ hipError_t launch_w4a8_mfma(const GemmArgs &a, int32_t *out, int num_cus, hipStr
 struct PromptTile {
   int tm = 0, wn = 0;
 };
+// Workgroups of mt x nt tiles, and the tile of one: workgroups go to the 8 XCDs in turn,
+// each XCD takes a contiguous run of tiles, in bands of four row tiles walked column by
+// column, so that the tiles it works on at one time (32 or more) form a block whose weights
+// are shared by four of them and whose activations by eight, in its L2. False past the
+// last tile.
+inline unsigned prompt_grid(int mt, int nt) { return 8u * (unsigned)(((size_t)mt * nt + 7) / 8); }
+__host__ __device__ inline bool prompt_tile(unsigned block, int mt, int nt, int &tm, int &tn) {
+  const int total = mt * nt, per = (total + 7) / 8;
+  const int t = (int)(block % 8) * per + (int)(block / 8);
+  if (t >= total || (int)(block / 8) >= per) return false;  // (its band may have no rows to divide by)
+  const int band = t / (4 * nt), in = t - band * 4 * nt, rows = mt - 4 * band < 4 ? mt - 4 * band : 4;
+  tn = in / rows;
+  tm = 4 * band + in - tn * rows;
+  return true;
+}
 // Whether a t16 GEMM of this shape runs faster on them than on the batch kernels, and how.
 bool prompt_tile_for(int fmt, int M, int N, int Kp, int num_cus, PromptTile *out);
 // W4A8 with many rows (lb_prompt.hip) on t16 weights and the quantizer's tiled (magic)

@@ -46,23 +46,10 @@ __device__ __forceinline__ void stage_ready() {
   __syncthreads();
 }
 
-// Tile of this workgroup: workgroups go to the 8 XCDs in turn, each XCD takes a
-// contiguous run of tiles, in bands of four row tiles walked column by column, so that
-// the tiles it works on at one time (32 or more) form a block whose weights are shared
-// by four of them and whose activations by eight, in its L2. False past the last tile.
-__device__ __forceinline__ bool prompt_tile(int mt, int nt, int &tm, int &tn) {
-  const int total = mt * nt, per = (total + 7) / 8;
-  const int t = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
-  const int band = t / (4 * nt), in = t - band * 4 * nt, rows = min(4, mt - 4 * band);
-  tn = in / rows;
-  tm = 4 * band + in - tn * rows;
-  return (int)(blockIdx.x / 8) < per && t < total;
-}
 template <typename Kern>
 static hipError_t launch_prompt(Kern kern, const GemmArgs &a, PromptTile t, hipStream_t s) {
   const int mt = (a.M + 16 * t.tm - 1) / (16 * t.tm), nt = (a.N + 64 * t.wn - 1) / (64 * t.wn);
-  const unsigned grid = 8u * (unsigned)(((size_t)mt * nt + 7) / 8);
-  hipLaunchKernelGGL(kern, dim3(grid), dim3(kPThreads), 0, s, a, mt, nt);
+  hipLaunchKernelGGL(kern, dim3(prompt_grid(mt, nt)), dim3(kPThreads), 0, s, a, mt, nt);
   return hipGetLastError();
 }
 
@@ -88,7 +75,7 @@ __global__ __launch_bounds__(kPThreads, 2) void w4a8_prompt_kernel(GemmArgs a, i
   const int q = lane >> 4, c = lane & 15;
   const int M = a.M, N = a.N, Kp = a.Kp, G = Kp / kGroup, G4 = t16_groups(Kp), S = (N + 15) / 16;
   int tm, tn;
-  if (!prompt_tile(mt, nt, tm, tn)) return;
+  if (!prompt_tile(blockIdx.x, mt, nt, tm, tn)) return;
   const int mb0 = tm * TM, s0 = (tn * kPWaves + wave) * WN;
   const uint32_t mblocks = (uint32_t)((M + 15) / 16);
   const Rsrc rx = make_rsrc(a.xq, mblocks * 16u * (uint32_t)Kp);
@@ -374,7 +361,7 @@ __global__ __launch_bounds__(kPThreads, 2) void mxfp4_prompt_kernel(GemmArgs a, 
   const int q = lane >> 4, c = lane & 15;
   const int M = a.M, N = a.N, Kp = a.Kp, G = (Kp + 127) / 128, G4 = t16_groups(Kp), S = (N + 15) / 16;
   int tm, tn;
-  if (!prompt_tile(mt, nt, tm, tn)) return;
+  if (!prompt_tile(blockIdx.x, mt, nt, tm, tn)) return;
   const int mb0 = tm * TM, s0 = (tn * kPWaves + wave) * WN;
   const uint32_t mblocks = (uint32_t)((M + 15) / 16);
   const uint32_t xbytes = mblocks * (uint32_t)G * (uint32_t)kDigitBlock;
@@ -648,7 +635,7 @@ __global__ __launch_bounds__(kPThreads, 2) void w4a16_prompt_kernel(GemmArgs a, 
   const int q = lane >> 4, c = lane & 15;
   const int M = a.M, N = a.N, Kp = a.Kp, G = Kp / kGroup, G4 = t16_groups(Kp), S = (N + 15) / 16;
   int tm, tn;
-  if (!prompt_tile(mt, nt, tm, tn)) return;
+  if (!prompt_tile(blockIdx.x, mt, nt, tm, tn)) return;
   const int mb0 = tm * TM, s0 = (tn * kPWaves + wave) * WN;
   const Rsrc rx = make_rsrc(a.x3, (uint32_t)min(x2h_bytes(M, Kp), (size_t)0xFFFFFFF0u));
   const Rsrc rw = make_rsrc(a.qw, (uint32_t)min(F8 ? t16f8_qw_bytes(N, Kp) : t16_qw_bytes(N, Kp), (size_t)0xFFFFFFF0u));

@@ -1,5 +1,5 @@
 """The load pipeline of the MXFP4 prompt GEMM in the code the compiler makes of it (CPU
-only: it compiles lb_prompt.hip to gfx950 assembly).
+only: it compiles lb_prompt.hip to gfx950 assembly), and the prompt GEMMs' tile map.
 
 The kernel waits for a stage by count: "all of this wave's loads but the last OPS have
 arrived". That holds only if the loads of an earlier group are issued before every load of
@@ -69,3 +69,17 @@ def test_no_step_waits_for_the_loads_it_issued(kernels):
             first = next(j for j in range(i, len(code)) if code[j].startswith("buffer_load"))
             waits = [int(n) for s in code[i - 4:first] for n in re.findall(r"vmcnt\((\d+)\)", s)]
             assert waits and min(waits) >= 8, (name, waits)
+
+
+def test_tile_map_covers_every_tile_once(tmp_path):
+    """Grids whose surplus workgroups fall past the last band of rows included: those must
+    be turned away before the band's row count (0) divides."""
+    cc = _hipcc()
+    if cc is None:
+        pytest.skip("hipcc not available")
+    exe = tmp_path / "prompt_tiles"
+    subprocess.run([cc, "--offload-host-only", "-x", "hip", "-O2", "-std=c++17", f"-I{_build.CSRC}",
+                    f"-I{_build.INCLUDE}", str(ROOT / "tests" / "csrc" / "prompt_tiles.hip"), "-o", str(exe)],
+                   check=True, capture_output=True, text=True)
+    r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0 and r.stdout == f"tiles {820 * 2485} bad 0\n", (r.returncode, r.stdout)
