@@ -177,6 +177,11 @@ typedef struct {
   int k_slices;          /* slices of 4096 elements each row is cut into, one wave each */
 } lbd_plan;
 int lbd_gemm_plan(int kind, int M, int N, int Kp, const lb_params *p, lbd_plan *out);
+/* 1 when the t16 GEMM of kind 0 = W4A16, 1 = MXFP4, 2 = W4A8 with this shape (and, for
+ * MXFP4, a workspace of lbd_bf16x3_workspace_bytes_split bytes, or NULL) runs as a prompt
+ * GEMM on the current device, with the rows and columns of Y its workgroups take, else 0;
+ * or LB_ERR_SHAPE / LB_ERR_ARG (a test hook, no reference counterpart) */
+int lbd_gemm_prompt_tile(int kind, int M, int N, int Kp, int *rows, int *cols);
 
 /* ---- MFMA tile layout ("t16") of int4 g128 weights (no reference counterpart:
  *      a device-private copy of an Int4Weights matrix, src/lowbit/formats.py:56-87,

@@ -525,6 +525,18 @@ int lbd_gemm_plan(int kind, int M, int N, int Kp, const lb_params *p, lbd_plan *
   return ok(out->path);
 }
 
+int lbd_gemm_prompt_tile(int kind, int M, int N, int Kp, int *rows, int *cols) {
+  static const int fmts[] = {lbk::F_W4A16, lbk::F_MXFP4, lbk::F_W4A8};
+  if (kind < 0 || kind > 2 || !rows || !cols) return fail(LB_ERR_ARG, "unknown GEMM kind or null pointer");
+  const int rc = check_shape(M, Kp, N, kind == 1 ? LB_MXBLOCK : LB_GROUP);
+  if (rc < 0) return rc;
+  lbk::PromptTile t;
+  const bool prompt = lbk::prompt_tile_for(fmts[kind], M, N, Kp, current_cus(), &t);
+  *rows = prompt ? 16 * t.tm : 0;
+  *cols = prompt ? 64 * t.wn : 0;
+  return ok(prompt ? 1 : 0);
+}
+
 int lbd_quantize_int4(const float *w, int N, int K, int asym, int signed_max, uint8_t *qw, float *scales,
                       uint8_t *zeros, void *stream) {
   if (N <= 0 || K <= 0) return fail(LB_ERR_SHAPE, "bad shape");

@@ -135,6 +135,7 @@ SIGNATURES = {
     "lbd_probe_grid_barrier": ([_int, _int, _int, _vp, _sz, _vp, _vp], _int),
     "lbd_gemm_path": ([_int, _int, _int, _pp], _int),
     "lbd_gemm_plan": ([_int, _int, _int, _int, _pp, C.c_void_p], _int),
+    "lbd_gemm_prompt_tile": ([_int, _int, _int, _int, C.POINTER(_int), C.POINTER(_int)], _int),
     "lbd_int4_t16_bytes": ([_int, _int, C.POINTER(_sz), C.POINTER(_sz), C.POINTER(_sz)], _int),
     "lbd_repack_int4_t16": ([_vp, _vp, _vp, _int, _int, _vp, _vp, _vp, _vp], _int),
     "lbd_gemm_w4a8_t16": ([_vp, _int, _int, _vp, _vp, _vp, _int, _vp, _pp, _vp, _sz, _vp], _int),
@@ -191,6 +192,15 @@ def gemm_plan(kind: str, m: int, n: int, kp: int, isa=None) -> dict:
     out = {f: getattr(p, f) for f, _ in LbdPlan._fields_}
     out["path"] = ISA_NAMES.get(p.path, "none")
     return out
+
+
+def prompt_tile(kind: str, m: int, n: int, kp: int):
+    """Rows and columns of Y that a workgroup takes where the t16 GEMM of this shape runs as
+    a prompt GEMM (lbd_gemm_prompt_tile), else None."""
+    rows, cols = C.c_int(), C.c_int()
+    rc = _check(lib().lbd_gemm_prompt_tile(KIND_IDS[kind], m, n, kp, C.byref(rows), C.byref(cols)),
+                "lbd_gemm_prompt_tile", False)
+    return (rows.value, cols.value) if rc else None
 
 
 class LbdFusion(C.Structure):

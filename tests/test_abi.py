@@ -169,6 +169,18 @@ def test_bf16x3_split_workspace_sizes():
         assert L.lbd_bf16x3_workspace_bytes_split(*args) == 0
 
 
+def test_prompt_tile_hook():
+    """Which t16 GEMMs run as prompt GEMMs (256 compute units assumed without a device)."""
+    assert K.prompt_tile("mxfp4", 777, 4096, 11008) == (32, 256) and K.prompt_tile("mxfp4", 200, 4096, 4096) == (16, 256)
+    assert K.prompt_tile("w4a16", 512, 4096, 4096) == (32, 256) and K.prompt_tile("w4a8", 2048, 11008, 4096) == (128, 128)
+    for kind in ("w4a16", "mxfp4", "w4a8"):
+        assert K.prompt_tile(kind, 32, 32768, 4096) is None and K.prompt_tile(kind, 64, 300, 1024) is None
+        with pytest.raises(ValueError):
+            K.prompt_tile(kind, 512, 4096, 100)
+    assert K.lib().lbd_gemm_prompt_tile(3, 512, 4096, 4096, C.byref(C.c_int()), C.byref(C.c_int())) == -6
+    assert K.lib().lbd_gemm_prompt_tile(0, 512, 4096, 4096, None, None) == -6
+
+
 def test_probe_argument_checks():
     """The measurement probes (lbd_probe_valu, lbd_empty_kernel, lbd_read_kernel,
     lbd_probe_grid_barrier) reject

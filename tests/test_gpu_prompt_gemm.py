@@ -15,9 +15,9 @@ from problems import outlier_int4_problem
 
 pytestmark = pytest.mark.gpu
 
-# M, N, K: ragged M and N, 1, 2, 3, 7 and 8 groups; 33 or more 16 x 16 tiles of Y per CU,
-# where every format takes these kernels
-SHAPES = [(1041, 3100, 128), (645, 5003, 256), (300, 9728, 384), (560, 4030, 896), (2090, 2601, 1024)]
+# M, N, K: ragged M and N, 1, 2, 3, 7 and 8 groups; 33 or more 16 x 16 tiles of Y per CU of
+# 256 (each test asserts that its shapes take these kernels, by the rows a workgroup takes)
+SHAPES = [(1041, 3100, 128), (645, 5003, 256), (300, 9728, 384), (2090, 2601, 1024)]
 
 
 def _int4(rng, n, k, asym, zmax=15):
@@ -27,9 +27,10 @@ def _int4(rng, n, k, asym, zmax=15):
                           rng.integers(0, zmax + 1, (n, g), dtype=np.uint8) if asym else None, k)
 
 
-@pytest.mark.parametrize("m,n,k", SHAPES)
+@pytest.mark.parametrize("m,n,k", SHAPES + [(560, 4030, 896)])
 @pytest.mark.parametrize("asym,zmax", [(False, 0), (True, 15), (True, 255)])
 def test_w4a8(rng, m, n, k, asym, zmax):
+    assert K.prompt_tile("w4a8", m, n, k)
     W = _int4(rng, n, k, asym, zmax)
     x = rng.standard_normal((m, k)).astype(np.float32)
     x[3] = 0
@@ -40,10 +41,57 @@ def test_w4a8(rng, m, n, k, asym, zmax):
     assert np.array_equal(y[3], np.zeros(n, np.float32))
 
 
-@pytest.mark.parametrize("m,n,k", SHAPES)
+# every tile height with 1, 3, 7, 8 and 9 groups
+W8_SHAPES = [(150, 2000, 128, 32), (300, 1500, 384, 32), (160, 4096, 896, 32), (200, 4096, 1152, 32),
+             (1041, 3100, 128, 64), (645, 5003, 384, 64), (256, 9728, 896, 64), (700, 4030, 1152, 64),
+             (1050, 6000, 128, 128), (1050, 6000, 384, 128), (512, 9728, 896, 128), (2090, 2601, 1024, 128)]
+
+
+@pytest.mark.parametrize("m,n,k,rows,zmax,wide", [
+    s + z for s in W8_SHAPES for z in ((15, False), (64, False), (255, False), (15, True)) if z[0] <= 64 or s[2] == 128])
+def test_w4a8_accumulators_are_exact(rng, m, n, k, rows, zmax, wide):
+    """With scales of +-1 a row of Y is an integer below 2^24 (9 groups of 128 x 127 x 64 at
+    the most; zero-points past 64 with K = 128 only) times the row's scale, rounded once.
+    wide: activations and codes at their extremes."""
+    assert K.prompt_tile("w4a8", m, n, k) == (rows, 128)
+    W = _int4(rng, n, k, True, zmax)
+    if zmax == 64:
+        W.zeros[::3] = 64
+    W.scales[:] = rng.choice([-1.0, 1.0], W.scales.shape)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    if wide:
+        x = np.sign(x).astype(np.float32)
+        W.qw[:] = rng.choice(np.array([0x00, 0xFF], np.uint8), W.qw.shape)
+        W.zeros[:] = rng.choice(np.array([0, 15], np.uint8), W.zeros.shape)
+    a = lb.quantize_act_int8(x)
+    w = W.codes().astype(np.float64) - np.repeat(W.zeros, 128, axis=1)
+    acc = a.xq.astype(np.float64) @ (w * np.repeat(W.scales, 128, axis=1)).T  # exact in float64
+    assert np.abs(acc).max() < 2 ** 24
+    np.testing.assert_array_equal(K.gemm_w4a8(x, lb.to_device(W)), acc.astype(np.float32) * a.scale[:, None])
+
+
+def test_w4a8_infinities_and_nan(rng):
+    """What row-major weights' kernel makes of them, and nothing in other rows."""
+    m, n, k = 645, 5003, 384
+    assert K.prompt_tile("w4a8", m, n, k)
+    W = _int4(rng, n, k, True)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    x[3, 7], x[20, 300], x[40], x[41, ::2] = np.inf, -np.inf, np.nan, np.nan
+    y, ref = K.gemm_w4a8(x, lb.to_device(W)), K.gemm_w4a8(x, W, isa="gfx950-mfma")
+    bad = ~np.isfinite(ref)
+    assert not bad[[i for i in range(m) if i not in (3, 20, 40, 41)]].any()
+    np.testing.assert_array_equal(y[bad], ref[bad])
+    a = lb.quantize_act_int8(np.where(np.isfinite(x), x, 0))
+    keep = np.isfinite(x).all(1)
+    _, bound = cref.c_gemm_w4a8(a.xq, a.scale, a.gsum, W.qw, W.scales, W.zeros)
+    assert (np.abs(y[keep] - ref[keep]) <= 2e-5 * bound[keep]).all()
+
+
+@pytest.mark.parametrize("m,n,k", SHAPES + [(500, 4030, 896), (384, 4099, 2176), (500, 4096, 3200)])
 @pytest.mark.parametrize("asym,zmax", [(False, 0), (True, 15), (True, 255)])
 def test_w4a16(rng, m, n, k, asym, zmax):
     """Zero-points past 15 rule the t16f8 copy out; elsewhere it gives t16's bits."""
+    assert K.prompt_tile("w4a16", m, n, k) == (32, 256)
     W = _int4(rng, n, k, asym, zmax)
     x = rng.standard_normal((m, k)).astype(np.float32)
     x[5] *= 1e30
@@ -61,9 +109,26 @@ def test_w4a16(rng, m, n, k, asym, zmax):
         np.testing.assert_array_equal(dy.to_array((m, n), np.float32), y)
 
 
+def test_w4a16_infinities_and_nan(rng):
+    """A row that holds one is NaN, as in the batch kernel; the others are as without it."""
+    m, n, k = 645, 5003, 384
+    assert K.prompt_tile("w4a16", m, n, k)
+    D = lb.to_device(_int4(rng, n, k, True))
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    y = K.gemm_w4a16(x, D)
+    x[3, 7], x[20, 300], x[41, ::2] = np.inf, -np.inf, np.nan
+    y2, keep = K.gemm_w4a16(x, D), np.isfinite(x).all(1)
+    assert np.isnan(y2[~keep]).all() and (~keep).sum() == 3
+    np.testing.assert_array_equal(y2[keep], y[keep])
+    batch = K.gemm_w4a16(x[:32], D)
+    assert K.prompt_tile("w4a16", 32, n, k) is None and np.isnan(batch[[3, 20]]).all()
+
+
 # MXFP4 also: a last group of one block; 16-row tiles with every number of groups left over
-@pytest.mark.parametrize("m,n,k", SHAPES + [(777, 4096, 1056), (200, 4100, 1152), (190, 4090, 1280), (235, 4089, 1408)])
-def test_mxfp4(rng, m, n, k):
+@pytest.mark.parametrize("m,n,k,rows", [s + (32,) for s in SHAPES + [(560, 4030, 896), (777, 4096, 1056)]] +
+                         [(200, 4100, 1152, 16), (190, 4090, 1280, 16), (235, 4089, 1408, 16)])
+def test_mxfp4(rng, m, n, k, rows):
+    assert K.prompt_tile("mxfp4", m, n, k) == (rows, 256)
     W = lb.MXFP4Weights(rng.integers(0, 256, (n, k // 2), dtype=np.uint8),
                         rng.integers(117, 131, (n, k // 32), dtype=np.uint8), k)
     W.e8m0[0], W.e8m0[1] = 0, 254  # the smallest and the largest scale
@@ -87,7 +152,8 @@ def test_mxfp4(rng, m, n, k):
 def test_columns_that_take_nothing_from_huge_elements(rng):
     """Where a row's few huge elements meet only zero weights, the other elements' products
     must keep the bound, which the huge ones then add nothing to."""
-    m, n, k = 640, 4096, 512
+    m, n, k = 512, 4096, 1152
+    assert K.prompt_tile("w4a16", m, n, k) and K.prompt_tile("mxfp4", m, n, k)
     x, W = outlier_int4_problem(rng, m, n, k)
     O.assert_fp_close(K.gemm_w4a16(x, lb.to_device(W)), O.gemm_w4a16_ref(x, W.qw, W.scales, W.zeros),
                       O.fp_bound(x, W.dequantize()), 1e-5)
@@ -102,8 +168,12 @@ def test_columns_that_take_nothing_from_huge_elements(rng):
         O.assert_fp_close(K.gemm_mxfp4(x, D), O.gemm_mxfp4_ref(x, W.qw, W.e8m0), O.fp_bound(x, W.dequantize()), 1e-5)
 
 
-# one 32-row and one 16-row tile shape (see lb_prompt.hip, prompt_tile_for)
+# one shape of 32-row tiles and one of 16-row ones
 MX_SHAPES = [(640, 4096, 512), (200, 4100, 1280)]
+
+
+def test_mxfp4_shapes_take_both_tiles():
+    assert [K.prompt_tile("mxfp4", *s) for s in MX_SHAPES] == [(32, 256), (16, 256)]
 
 
 def _mx_limit(x, W, y):
@@ -138,20 +208,23 @@ def test_mxfp4_activation_magnitudes(rng, m, n, k, mag):
     assert _mx_limit(x, W, K.gemm_mxfp4(x, lb.to_device(W))) <= 1.0
 
 
-@pytest.mark.parametrize("m,n,k", MX_SHAPES)
+@pytest.mark.parametrize("m,n,k", MX_SHAPES + [(528, 4100, 8320), (200, 4100, 8320)])  # 65 groups too
 @pytest.mark.parametrize("mag", [1e-20, 1.0, 1e30])
 def test_mxfp4_keeps_every_bit_of_an_activation(rng, m, n, k, mag):
-    """Weight rows with a single 1: y[i, j] is the activation x[i, j % k] itself, normal or
+    """Weight rows with a single 1: y[i, j] is one of row i's activations itself, normal or
     log-uniform over 2^40, whatever its neighbours are. (All above 2^-110: below it the last
     of an activation's three bf16 terms would be a subnormal, which the matrix cores flush,
     2^-16 of the element at the most, in the batch kernel as here.)"""
+    assert K.prompt_tile("mxfp4", m, n, k)
     x = rng.standard_normal((m, k)).astype(np.float32)
     x[m // 2:] *= np.exp2(rng.uniform(-20, 20, x[m // 2:].shape)).astype(np.float32)
     x *= np.float32(mag)
     codes = np.zeros((n, k), np.uint8)
-    codes[np.arange(n), np.arange(n) % k] = 2  # E2M1 1.0
+    col = np.arange(n) % k
+    col[::2] = k - 1 - col[::2]
+    codes[np.arange(n), col] = 2  # E2M1 1.0
     W = lb.MXFP4Weights(lb.formats.pack_nibbles(codes, 32), np.full((n, k // 32), 127, np.uint8), k)
-    np.testing.assert_array_equal(K.gemm_mxfp4(x, lb.to_device(W)), x[:, np.arange(n) % k])
+    np.testing.assert_array_equal(K.gemm_mxfp4(x, lb.to_device(W)), x[:, col])
 
 
 @pytest.mark.parametrize("m,n,k", MX_SHAPES)
@@ -177,6 +250,7 @@ def test_mxfp4_y_on_x(rng, shift):
     """Y may lie on X (N = K), or begin in X's last row: marked blocks are read from X while
     Y is stored, so such a call takes the batch kernel, which is done with X by then."""
     m, n = 1040, 2048
+    assert K.prompt_tile("mxfp4", m, n, n)
     W = lb.quantize_mxfp4(rng.standard_normal((n, n)).astype(np.float32))
     x = rng.standard_normal((m, n)).astype(np.float32)
     x[:, ::9] *= 1e9
