@@ -1363,6 +1363,12 @@ bool w4a16_prefers_t16f8(int M, int N, int Kp, int num_cus) {
   // stage cost more than the conversions it saves when cold (5-13 % more time). At 64
   // x 4096 x 11008 split in two (4 subtiles) t16f8 took 27.2 against 30.2 us hot, 32.1
   // against 32.3 cold; 128 x 4096 x 11008 unsplit (4), 43.3 against 49.6 hot.
+  // The prompt GEMM gains from t16f8 (512 x 4096 x 4096 46.9 against 53.6, 33 x 151936 x 896
+  // 45.6 against 49.1, 64 x 32768 x 4096 44.8 against 48.8) until its bytes, one a weight, no
+  // longer stay in the 256 MiB last-level cache (64 x 32768 x 8192 108.7 against 90.1, 48 x
+  // 151936 x 2048 105 against 86, 384 x 32768 x 11008 542 against 512).
+  PromptTile tile;
+  if (prompt_tile_for(F_W4A16, M, N, Kp, num_cus, &tile)) return t16f8_qw_bytes(N, Kp) < ((size_t)256 << 20);
   int gx, gy, spw;
   const int cus = num_cus > 0 ? num_cus : 256;
   bf3_grid(M, N, M > 16 ? 2 : 1, cus, gx, gy, spw);

@@ -147,6 +147,9 @@ def test_t16_sizes_and_argument_checks():
     # at K = 11008 the split launch counts: 64 rows split in two give 4 subtiles per workgroup
     assert L.lbd_w4a16_prefers_t16f8(64, 4096, 11008) == 1 and L.lbd_w4a16_prefers_t16f8(0, 16, 128) == -1
     assert L.lbd_w4a16_prefers_t16f8(16, 4096, 11008) == 0 and L.lbd_w4a16_prefers_t16f8(32, 4096, 11008) == 0
+    # prompt GEMMs: t16f8 while its bytes (one a weight) are below 256 MiB
+    assert L.lbd_w4a16_prefers_t16f8(512, 4096, 4096) == 1 and L.lbd_w4a16_prefers_t16f8(64, 32768, 4096) == 1
+    assert L.lbd_w4a16_prefers_t16f8(64, 32768, 8192) == 0 and L.lbd_w4a16_prefers_t16f8(48, 151936, 2048) == 0
     assert L.lbd_gemm_path(2, 1, 4096, C.byref(prm)) == K.ISA_GFX950
     assert L.lbd_gemm_path(2, 64, 4096, C.byref(prm)) == K.ISA_GFX950_MFMA
     assert L.lbd_gemm_path(7, 1, 4096, C.byref(prm)) == -6
