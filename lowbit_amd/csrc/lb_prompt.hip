@@ -801,6 +801,8 @@ hipError_t launch_w4a16_prompt(const GemmArgs &a, PromptTile t, bool f8, hipStre
 //          when the chip is full, against 0.0235 T a group of the batch kernel, which
 //          works on phases of 32 groups (1024 x 4096 x 11008 231 -> 90, 384 x 4096 x 1024
 //          22.9 -> 12.4, 2048 x 11008 x 4096 252 -> 150; 256 x 4096 x 4096 17.8 against 25).
+//          One whole phase is the batch kernel at its best (256 x 9728 x 4096 32.6 against
+//          34.2, not taken; 384 x 9728 x 4096 44.1 -> 35.1).
 // Few rows (32 and less) stay with the batch kernels, which are built for them.
 bool prompt_tile_for(int fmt, int M, int N, int Kp, int num_cus, PromptTile *out) {
   if (M <= 32) return false;
@@ -823,7 +825,8 @@ bool prompt_tile_for(int fmt, int M, int N, int Kp, int num_cus, PromptTile *out
     const double per[3] = {std::max(0.57, 0.0205 * T), std::max(0.72, 0.0163 * T), std::max(1.13, 0.0140 * T)};
     const int best = (int)(std::min_element(per, per + 3) - per);
     t = PromptTile{2 << best, 2};
-    if (1.0 + G * per[best] > 0.9 * 0.0235 * T * 32 * std::ceil(G / 32)) return false;
+    const double batch = 0.0235 * T * 32 * std::ceil(G / 32);
+    if (1.0 + G * per[best] > (G == 32 ? 0.8 : 0.9) * batch) return false;
   } else {
     return false;
   }
