@@ -50,6 +50,8 @@ INT8_PEAK_TOPS = 5000.0      # dense int8 MFMA, published (POP/s -> TOP/s here)
 FP32_PEAK_TFLOPS = 157.3     # dense fp32 matrix, published
 BF16_PEAK_TFLOPS = 2500.0    # dense bf16 MFMA, published
 BF16X3_TERMS = 3             # bf16 products per fp32 product on the bf16x3 path (MXFP4)
+MX_PEAK_TFLOPS = 10000.0     # dense MXFP6 / MXFP4, published
+MX_DIGITS = 8                # six-bit products per product in MXFP4's prompt GEMM
 F16X2_TERMS = 2              # float16 products per product on the W4A16 two-term path
 COLD_POOL_BYTES = 1280 << 20  # > 2 x (256 MB MALL + 32 MB L2)
 DECODE = (1, 11008, 4096)
@@ -1007,6 +1009,9 @@ def main() -> int:
                 terms = F16X2_TERMS if fmt == "w4a16" else BF16X3_TERMS
                 r["mfma"] = "f16x2" if fmt == "w4a16" else "bf16x3"
                 r["mfma_frac"] = round(terms * r["gflops"] / 1e3 / BF16_PEAK_TFLOPS, 4)
+                if fmt == "mxfp4" and dev.K.prompt_tile(fmt, mb, nb, W.kp):
+                    r["mfma"] = "fp6x8"
+                    r["mfma_frac"] = round(MX_DIGITS * r["gflops"] / 1e3 / MX_PEAK_TFLOPS, 4)
                 r["fp32_equiv_frac"] = round(r["gflops"] / 1e3 / FP32_PEAK_TFLOPS, 4)
             else:
                 r["mfma"] = "fp32"

@@ -202,7 +202,9 @@ int lbd_repack_int4_t16(const uint8_t *qw, const float *scales,
                         const uint8_t *zeros, int N, int Kp, uint8_t *qwt,
                         float *st, uint8_t *zt, void *stream);
 /* y = x . w^T as lbd_gemm_w4a8 (same workspace contract), weights in the t16
- * layout; always the int8 matrix-core path (returns LB_ISA_GFX950_MFMA) */
+ * layout; always the int8 matrix-core path (returns LB_ISA_GFX950_MFMA). The same bits as
+ * row-major weights give there, except with many rows (lbd_gemm_prompt_tile), where the
+ * exact group sums are scaled and added in another order, within the same bound */
 int lbd_gemm_w4a8_t16(const float *x, int M, int Kp, const uint8_t *qwt,
                       const float *st, const uint8_t *zt, int N, float *y,
                       const lb_params *p, void *workspace,

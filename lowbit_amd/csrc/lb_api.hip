@@ -808,6 +808,7 @@ int lbd_qkv_rope(float *qkv, const float *bias, int T, int H, int KV, int D, con
             "qkv rope launch");
 }
 
+// cap <= 16000: the caches' range in every attention call, not a limit of this kernel.
 int lbd_attention(const float *q, int qstride, const float *k_cache, const float *v_cache, int T, int H, int KV, int D,
                   const int32_t *pos, int cap, float *out, void *stream) {
   if (T <= 0 || H <= 0 || KV <= 0 || H % KV || (D != 32 && D != 64 && D != 128) || cap <= 0 || cap > 16000 ||

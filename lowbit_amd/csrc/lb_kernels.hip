@@ -60,7 +60,8 @@ __device__ __forceinline__ uint32_t w4a8_tiled_offset(int m, int e, int G) {
 // pieces share cache lines, are given to one XCD, whose L2 puts the lines together (whole
 // GEMMs: W4A16 512 x 4096 x 4096 48.9 -> 46.1 us, W4A8 1000 x 4096 x 11008 91.7 -> 84.6).
 // Up to 112 rows the grid stays exact, without the two instructions: too few lines for it to
-// matter (W4A8 64 x 11008 x 4096 12.14 against 12.24 us with it).
+// matter (W4A8 64 x 11008 x 4096 12.14 against 12.24 us with it). Ahead of the W4A8 prompt
+// GEMM it is taken at any number of rows.
 constexpr int kRowsInTurn = 112;
 __device__ __forceinline__ int row_of_block(int b) { return (b & ~127) | ((b & 7) << 4) | ((b >> 3) & 15); }
 static unsigned row_grid(int M) { return (unsigned)((M + 127) / 128 * 128); }

@@ -57,8 +57,8 @@ static hipError_t launch_prompt(Kern kern, const GemmArgs &a, PromptTile t, hipS
 //
 // The exact int32 group accumulators come out of the int8 MFMAs as float bits: the
 // first product's C operand is the bit pattern of 1.5 * 2^23 (whose unit is 1), so the
-// accumulator 1.5 * 2^23 + sum, |sum| < 2^18, is that float's bit pattern plus an
-// integer, i.e. the float 12582912 + sum exactly. One subtraction (a full-rate
+// accumulator 1.5 * 2^23 + sum, |sum| <= 128 x 127 x 64 < 2^20, is that float's bit pattern
+// plus an integer, i.e. the float 12582912 + sum exactly. One subtraction (a full-rate
 // instruction, unlike an int conversion) and one FMA with the group scale per output.
 // Codes enter as q - z + 64 (a positive byte for z <= 64: no borrow between bytes); the
 // activations' group sums, times -64, are part of the C operand (kPromptMagic - 64 asum,
@@ -787,13 +787,15 @@ hipError_t launch_w4a16_prompt(const GemmArgs &a, PromptTile t, bool f8, hipStre
 // a launch that leaves each CU one workgroup or less takes (a little more than) G times
 // its time per group however few rows there are, while the batch kernels' time falls with
 // the work; so the line is drawn in 16 x 16 tiles of Y per CU, T.
-//   MXFP4  about 11 us + 0.68 a group with 16-row tiles, taken while they fill one round of
-//          the CUs, 12.5 + 0.97 a group and round with 32-row ones, against 8 us + 1.0-1.1 a
-//          group of the batch kernel up to T = 22, 1.5 at 24, 0.06 T above (normal activations
-//          with a few large channels): 192 x 4096 x 4096 40.7 -> 32.2, 448 x 4096 x 4096
-//          64.5 -> 46.1, 1024 x 4096 x 4096 179 -> 80, 33 x 28672 x 8192 93.3 -> 72.5, 1024
-//          x 4096 x 11008 448 -> 187. Not taken: 192 x 4096 x 1024 15.4 against 16.3, 112 x
-//          11008 x 4096 (T = 19) 40.3 against 44.3, 208 x 9728 x 896 (T = 31) 20.6 against 24.2.
+//   MXFP4  11 us + 0.68 a group with 16-row tiles, taken while they fill one round of the CUs;
+//          12.5 + 0.97 a group with 32-row ones in one round, 1 + r / 2 in r <= 2, r + 0.6 in
+//          more; against 8 us + (0.5 + 0.0002 M) a group and chunk of the batch kernel, a chunk
+//          being 6 of the 16-column subtiles that a workgroup of its grid walks (normal
+//          activations with a few large channels; 170 shapes of 33-1552 rows): 192 x 4096 x
+//          4096 40.7 -> 32.2, 448 x 4096 x 4096 64.5 -> 46.1, 1024 x 4096 x 4096 179 -> 80,
+//          33 x 28672 x 8192 93.3 -> 72.5, 1024 x 4096 x 11008 448 -> 187. Not taken: 192 x
+//          4096 x 1024 15.4 against 16.3, 112 x 11008 x 4096 40.3 against 44.3, 240 x 9085 x
+//          7008 98.1 against 101, 272 x 8013 x 2048 35.9 against 41.0.
 //   W4A16  1.13 us a group and round of 256 workgroups against 0.055 T of the batch kernel
 //          (512 x 4096 x 4096 60.5 -> 49.0, 2048 x 11008 x 4096 642 -> 364; 256 x 4096 x
 //          4096 39.9 against 44.4, not taken).
@@ -816,8 +818,10 @@ bool prompt_tile_for(int fmt, int M, int N, int Kp, int num_cus, PromptTile *out
   PromptTile t;
   if (fmt == F_MXFP4) {
     t = PromptTile{rounds(1, 4) <= 1 ? 1 : 2, 4};
-    const bool gains = t.tm == 1 ? T >= 12 && G >= 9 : T >= 33 || (T >= 24 && G >= 8) || (T >= 17 && G >= 64);
-    if (!gains) return false;
+    const double r = rounds(2, 4), per = t.tm == 1 ? 0.68 : r <= 1 ? 0.97 : r <= 2 ? 1 + 0.5 * r : r + 0.6;
+    const int gy = (M + 31) / 32, S = (N + 15) / 16, gx = std::max(1, std::min(S, (int)cus / gy));
+    const double chunks = ((S + gx - 1) / gx + 5) / 6;
+    if ((t.tm == 1 ? 11 : 12.5) + G * per > 0.97 * (8 + G * chunks * (0.5 + 0.0002 * M))) return false;
   } else if (fmt == F_W4A16) {
     t = PromptTile{2, 4};
     if (1.13 * std::ceil(rounds(2, 4)) > 0.055 * T) return false;

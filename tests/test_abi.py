@@ -176,6 +176,9 @@ def test_prompt_tile_hook():
     """Which t16 GEMMs run as prompt GEMMs (256 compute units assumed without a device)."""
     assert K.prompt_tile("mxfp4", 777, 4096, 11008) == (32, 256) and K.prompt_tile("mxfp4", 200, 4096, 4096) == (16, 256)
     assert K.prompt_tile("w4a16", 512, 4096, 4096) == (32, 256) and K.prompt_tile("w4a8", 2048, 11008, 4096) == (128, 128)
+    # MXFP4: the batch kernel where its grid comes out even, or K is short
+    assert K.prompt_tile("mxfp4", 240, 9085, 7008) is None and K.prompt_tile("mxfp4", 240, 10093, 7008) == (32, 256)
+    assert K.prompt_tile("mxfp4", 192, 4096, 1024) is None and K.prompt_tile("mxfp4", 112, 11008, 4096) is None
     # one whole phase of 32 groups: the batch kernel is as fast until there are more tiles
     assert K.prompt_tile("w4a8", 256, 9728, 4096) is None and K.prompt_tile("w4a8", 384, 9728, 4096) == (64, 128)
     for kind in ("w4a16", "mxfp4", "w4a8"):

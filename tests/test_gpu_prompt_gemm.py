@@ -124,8 +124,9 @@ def test_w4a16_infinities_and_nan(rng):
     assert K.prompt_tile("w4a16", 32, n, k) is None and np.isnan(batch[[3, 20]]).all()
 
 
-# MXFP4 also: a last group of one block; 16-row tiles with every number of groups left over
-@pytest.mark.parametrize("m,n,k,rows", [s + (32,) for s in SHAPES + [(560, 4030, 896), (777, 4096, 1056)]] +
+# 1, 2, 3, 7, 8 and 9 groups, the last of one block; 16-row tiles with every number left over
+@pytest.mark.parametrize("m,n,k,rows", [s + (32,) for s in [(2090, 6003, 128), (2090, 5003, 256), (900, 9728, 384),
+                                                            (700, 4030, 896), (2090, 2601, 1024), (777, 4096, 1056)]] +
                          [(200, 4100, 1152, 16), (190, 4090, 1280, 16), (235, 4089, 1408, 16)])
 def test_mxfp4(rng, m, n, k, rows):
     assert K.prompt_tile("mxfp4", m, n, k) == (rows, 256)
@@ -169,7 +170,7 @@ def test_columns_that_take_nothing_from_huge_elements(rng):
 
 
 # one shape of 32-row tiles and one of 16-row ones
-MX_SHAPES = [(640, 4096, 512), (200, 4100, 1280)]
+MX_SHAPES = [(1300, 4096, 512), (200, 4100, 1280)]
 
 
 def test_mxfp4_shapes_take_both_tiles():
