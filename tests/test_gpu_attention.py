@@ -33,7 +33,11 @@ def draw(rng, T, H, KV, D, cap):
 @pytest.mark.parametrize("D", [32, 64, 128])
 @pytest.mark.parametrize("T,H,KV,pos,cap,shift", [
     (1, 2, 1, 0, 1, 0), (16, 3, 1, 0, 16, 1), (17, 4, 2, 15, 40, 2), (32, 2, 2, 0, 32, 0), (33, 7, 1, 31, 64, 3),
-    (47, 2, 1, 513, 561, 0), (65, 4, 4, 0, 65, 1), (20, 2, 1, 1080, 1100, 0)])
+    (47, 2, 1, 513, 561, 0), (65, 4, 4, 0, 65, 1), (20, 2, 1, 1080, 1100, 0),
+    # caches of 48 positions and less have a kernel of their own: its last size, and the
+    # tiles' edges above it
+    (48, 3, 1, 0, 48, 1), (5, 2, 1, 43, 48, 0), (49, 3, 1, 0, 49, 1), (1, 2, 1, 0, 49, 0), (16, 3, 1, 0, 64, 1),
+    (17, 4, 2, 15, 50, 2), (32, 2, 2, 0, 64, 0), (33, 4, 2, 15, 49, 3)])
 def test_tile_edges(rng, D, T, H, KV, pos, cap, shift):
     q, kc, vc = draw(rng, T, H, KV, D, cap)
     kc[:, pos + T:], vc[:, pos + T:] = np.nan, np.nan  # cache rows past the keys in use
@@ -44,11 +48,12 @@ def test_tile_edges(rng, D, T, H, KV, pos, cap, shift):
 
 @pytest.mark.parametrize("D", [32, 64, 128])
 @pytest.mark.parametrize("bad", [np.nan, np.inf, -np.inf])
-def test_rows_a_query_does_not_see_may_hold_anything(rng, D, bad):
+@pytest.mark.parametrize("cap", [48, 80])
+def test_rows_a_query_does_not_see_may_hold_anything(rng, D, bad, cap):
     """Key 21's value (then key 38's key) is not finite: queries before it are the
     finite attention, queries from it on are not finite (NaN scores and sums)."""
     T, H, KV, pos = 45, 4, 2, 3
-    q, kc, vc = draw(rng, T, H, KV, D, pos + T)
+    q, kc, vc = draw(rng, T, H, KV, D, cap)
     ref = attention_ref(q[:, :H * D].reshape(T, H, D), kc, vc, pos, H, KV)
     v2 = vc.copy()
     v2[:, 21] = bad
