@@ -303,10 +303,12 @@ __global__ __launch_bounds__(NW *kWave) void attention_kernel(const float *__res
 // The same over a cache of few positions: one workgroup of one wave per (token, head),
 // scores one key per lane into LDS, wave max and sum, then lane l owns output elements
 // l, l + 64, ... below D. Bound by latency, which a wave for each query and head keeps
-// shorter than 16 queries on the matrix cores: 16 heads on 4, D = 128, 30 tokens 5.53 -> 4.38
-// us, 48 tokens 6.21 -> 5.15; D = 32 and 64 4.35 -> 4.1. From 64 tokens at 32 heads, and for
-// all from 100, the kernel above is the faster (D = 64, 14 heads, 384 tokens 10.4 against 51).
-constexpr int kShortCache = 48;
+// shorter than 16 queries on the matrix cores while the keys are few and so are the waves:
+// caches of 64 positions (one key a lane; 104 at D = 128, whose products take longer there) and
+// 51000 scores, rows past the keys in use counted. D = 128: 16 heads on 4, 30 tokens 5.53 ->
+// 4.38 us, 56 6.27 -> 5.99 (64 6.61 against 7.12, not taken); 8 heads, 64 tokens 6.60 -> 5.40,
+// 52 behind 40 8.01 -> 7.38; one head, 96 tokens 7.57 -> 7.16; D = 32 and 64 4.5 -> 4.2.
+constexpr long long kShortScores = 51000;
 template <int D>
 __global__ __launch_bounds__(kWave) void attention_short_kernel(const float *__restrict__ q, int qstride,
                                                                 const float *__restrict__ kc,
@@ -719,7 +721,7 @@ hipError_t launch_attention(const float *q, int qstride, const float *kc, const 
                        cap, out);
     return hipGetLastError();
   };
-  if (cap <= kShortCache && H <= 65535) {
+  if (cap <= (D == 128 ? 104 : 64) && (long long)T * H * cap <= kShortScores) {
     if (D == 32) return go_short(attention_short_kernel<32>);
     if (D == 64) return go_short(attention_short_kernel<64>);
     if (D == 128) return go_short(attention_short_kernel<128>);

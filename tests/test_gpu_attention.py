@@ -34,10 +34,11 @@ def draw(rng, T, H, KV, D, cap):
 @pytest.mark.parametrize("T,H,KV,pos,cap,shift", [
     (1, 2, 1, 0, 1, 0), (16, 3, 1, 0, 16, 1), (17, 4, 2, 15, 40, 2), (32, 2, 2, 0, 32, 0), (33, 7, 1, 31, 64, 3),
     (47, 2, 1, 513, 561, 0), (65, 4, 4, 0, 65, 1), (20, 2, 1, 1080, 1100, 0),
-    # caches of 48 positions and less have a kernel of their own: its last size, and the
-    # tiles' edges above it
-    (48, 3, 1, 0, 48, 1), (5, 2, 1, 43, 48, 0), (49, 3, 1, 0, 49, 1), (1, 2, 1, 0, 49, 0), (16, 3, 1, 0, 64, 1),
-    (17, 4, 2, 15, 50, 2), (32, 2, 2, 0, 64, 0), (33, 4, 2, 15, 49, 3)])
+    # few scores over at most 64 positions (104 at D = 128) have a kernel of their own: its last
+    # sizes, and the tiles' edges past it
+    (64, 12, 4, 0, 64, 1), (64, 13, 1, 0, 64, 0), (5, 2, 1, 59, 64, 0), (40, 3, 1, 64, 104, 1), (33, 32, 4, 16, 49, 1),
+    (1, 2, 1, 0, 105, 0), (16, 3, 1, 0, 112, 1), (17, 4, 2, 88, 105, 2), (32, 2, 2, 0, 128, 0), (33, 7, 1, 72, 105, 3),
+    (48, 3, 1, 60, 120, 1), (65, 4, 4, 41, 106, 1)])
 def test_tile_edges(rng, D, T, H, KV, pos, cap, shift):
     q, kc, vc = draw(rng, T, H, KV, D, cap)
     kc[:, pos + T:], vc[:, pos + T:] = np.nan, np.nan  # cache rows past the keys in use
@@ -48,7 +49,7 @@ def test_tile_edges(rng, D, T, H, KV, pos, cap, shift):
 
 @pytest.mark.parametrize("D", [32, 64, 128])
 @pytest.mark.parametrize("bad", [np.nan, np.inf, -np.inf])
-@pytest.mark.parametrize("cap", [48, 80])
+@pytest.mark.parametrize("cap", [48, 120])
 def test_rows_a_query_does_not_see_may_hold_anything(rng, D, bad, cap):
     """Key 21's value (then key 38's key) is not finite: queries before it are the
     finite attention, queries from it on are not finite (NaN scores and sums)."""
