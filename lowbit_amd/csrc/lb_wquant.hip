@@ -25,23 +25,32 @@ namespace lbk {
 // the group's lanes by DPP within a row of 16. (With two elements per lane, 4-byte loads,
 // 1-byte stores and a permute per reduction step, int4 asym 4096 x 11008 took 88.6 us and
 // MXFP4 121.8; now 45.3 and 40.1, against 41 us for the bytes at a large copy's rate.)
-// Rows that are not 16-byte aligned (K % 4, or the pointers) load and store element by
-// element (VEC false).
+// Rows that are not 16-byte aligned (VEC false: K % 4, or the pointers) take the same loads
+// at any float's address, element by element only where the row ends inside one, and store
+// bytes only where qw itself is not aligned (each element loaded and each byte stored by
+// itself, int4 groups of 32 at 4096 x 1001 took 9.3 us, and 7.6 before the lanes held four
+// elements; now 5.1).
 constexpr int kQT = 256;  // 4 waves per workgroup
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
 
 template <bool VEC>
 __device__ __forceinline__ void load4(const float *wr, int k, int K, bool live, float (&x)[4]) {
   if constexpr (VEC) {
     const float4 t = live && k < K ? *reinterpret_cast<const float4 *>(wr + k) : make_float4(0.f, 0.f, 0.f, 0.f);
     x[0] = t.x, x[1] = t.y, x[2] = t.z, x[3] = t.w;
+  } else if (live && k + 4 <= K) {
+    const f4u t = *reinterpret_cast<const f4u *>(wr + k);
+#pragma unroll
+    for (int i = 0; i < 4; i++) x[i] = t[i];
   } else {
 #pragma unroll
     for (int i = 0; i < 4; i++) x[i] = live && k + i < K ? wr[k + i] : 0.0f;
   }
 }
 template <bool VEC>
-__device__ __forceinline__ void store4(uint8_t *dst, uint32_t v) {
-  if constexpr (VEC) {
+__device__ __forceinline__ void store4(uint8_t *qw, size_t off, uint32_t v) {  // off % 4 == 0
+  uint8_t *dst = qw + off;
+  if (VEC || reinterpret_cast<uintptr_t>(qw) % 4 == 0) {
     *reinterpret_cast<uint32_t *>(dst) = v;
   } else {
 #pragma unroll
@@ -128,7 +137,7 @@ __global__ __launch_bounds__(kQT) void quantize_int4_kernel(const float *__restr
     bytes |= (uint32_t)c << (8 * (i & 3) + 4 * (i >> 2));
   }
   if (!live) return;
-  store4<VEC>(qw + (size_t)row * ((size_t)G * (GS / 2)) + (size_t)g * (GS / 2) + 4 * j, bytes);
+  store4<VEC>(qw, (size_t)row * ((size_t)G * (GS / 2)) + (size_t)g * (GS / 2) + 4 * j, bytes);
   if (j == 0) {
     scales[(size_t)row * G + g] = s;
     if (MODE == 2) zeros[(size_t)row * G + g] = (uint8_t)pad;
@@ -190,7 +199,7 @@ __global__ __launch_bounds__(kQT) void quantize_mxfp4_kernel(const float *__rest
 #pragma unroll
   for (int i = 0; i < 8; i++) bytes |= e2m1_code(x[i >> 2][i & 3] * inv) << (8 * (i & 3) + 4 * (i >> 2));
   const int nb = Kp / 32;
-  store4<VEC>(qw + (size_t)row * (Kp / 2) + blk * 16 + 4 * j, bytes);
+  store4<VEC>(qw, (size_t)row * (Kp / 2) + blk * 16 + 4 * j, bytes);
   if (j == 0) e8m0[(size_t)row * nb + blk] = (uint8_t)e;
 }
 
