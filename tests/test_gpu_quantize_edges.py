@@ -1,6 +1,7 @@
 """The weight quantizers' load paths (GPU), byte for byte against the host packers: 16-byte
-loads where K % 4 == 0, element loads elsewhere and from unaligned pointers, rows that end
-inside a wave's 512 elements and inside either half of a group."""
+loads of aligned rows (K % 4 == 0) and at any float's address elsewhere, rows that end inside
+such a load, inside a wave's 512 elements and inside either half of a group, and byte stores
+to an unaligned packed array."""
 import numpy as np
 import pytest
 
