@@ -240,7 +240,7 @@ size_t lbd_bf16x3_workspace_bytes(int M, int Kp);
  * lbd_bf16x3_workspace_bytes the unsplit GEMM; both meet the same bound, not the
  * same bits. (W4A16 shapes of many rows that run as prompt GEMMs take no split and leave
  * the room for it unused.) MXFP4 shapes of many rows that run as prompt GEMMs with this
- * size, and as the batch kernel with lbd_bf16x3_workspace_bytes, take 1/48 more than the
+ * size, and as the batch kernel with lbd_bf16x3_workspace_bytes, take 2 % more than the
  * latter. Elsewhere it equals lbd_bf16x3_workspace_bytes rounded up to 256; 0 for an
  * invalid argument. (No reference counterpart: the reference's GEMMs take no workspace.) */
 size_t lbd_bf16x3_workspace_bytes_split(int kind, int M, int N, int Kp);

@@ -258,6 +258,11 @@ hipError_t launch_w4a8_prompt(const GemmArgs &a, PromptTile t, hipStream_t s) {
 // a large one. Marks on every loss take 80 % of the 16-row groups of normal activations with
 // seven digits, 5 % with eight.)
 //
+// Measured at 777 x 4096 x 11008, the bf16 batch kernel taking 336 us: 146 us with no marked
+// block, 169 for normal activations, 173 with a few channels 8 times the rest, 175 and 182
+// with four channels 128 and 512 times the rest (2048 x 11008 x 4096: 306, 367, 368, 398, 428
+// against 837). The digits' products bound it, the split takes 17 of it.
+//
 // Digit tile of (row block, group, digit): lane 16 q + c holds row c, block 4 g + q, slots
 // 2 j / 2 j + 1 = elements j / j + 16 (the nibbles of byte j of the packed weights),
 // 24 bytes as 16 (1 KiB for the wave) then 8 (512 B), row blocks within a group. After all
